@@ -60,6 +60,8 @@ struct oc_dg
   // bumped by every setter that replaces device data a captured graph may hold
   uint64_t generation = 0;
   unsigned int *d_sweeps_blk = nullptr;
+  double *d_eig = nullptr;  // FP64 wet depth solve: OpArgs::eig
+  double eig_sum = 0.0, eig_min = 0.0;
   float *d_jmat = nullptr;  // mixed precision: closed-form Jacobi matrix (unit cell)
   float *d_kinv = nullptr;  // mixed precision: momentum inverse mass (unit cell)
   unsigned long long *d_defer = nullptr;  // mixed precision: per batch, deferred lanes
@@ -116,6 +118,9 @@ struct oc_dg
     o.has_coriolis = (d_cell0[4] != nullptr) || (c_cell0[4] != 0.0);
     o.max_it = max_it;
     o.xcd_swizzle = xcd_swizzle;
+    o.eig = d_eig;
+    o.eig_sum = eig_sum;
+    o.eig_min = eig_min;
     o.jmat = d_jmat;
     o.kinv = d_kinv;
     o.wet_margin = wet_margin;

@@ -38,6 +38,9 @@ struct Basis
   R M1[MAXN1][MAXN1];        // sum_a Sg[a][i] Sg[a][j] wg[a]: 1-D GL(ng) mass (exact)
   R Sn[MAXN1][MAXN1];        // l_i at Gauss(n1) points (velocity projection)
   R Psub[2][MAXN1][MAXN1];   // l_k((x_j + s)/2), x_j the nodes: restriction to half s
+  // 1-D eigenvectors of D1^-1 M1 (D1 the lumped mass): M1 = D1 Ve diag(el) Ved, with Ved =
+  // Ve^-1 D1^-1, so that (Ved x Ved) r are the eigen-coefficients of D^-1 r on the unit cell
+  R Ve[MAXN1][MAXN1], Ved[MAXN1][MAXN1];
   R lam;                     // max_{a,i} Sg[a][i]^2: bound of |phi_ij| at the GL(ng)^2 points
 };
 using DegreeTables = Basis<double>;
@@ -84,6 +87,11 @@ struct OpArgs
   // mixed precision: closed form of max_it linear Jacobi sweeps on a wet unit cell,
   // [nd][nd] row-major (delta = J r / area), and the wet-cell safety factor
   const float *jmat;
+  // the capped sweeps of a wet cell in the eigenbasis of D^-1 M (wet_depth_solve): per
+  // eigen-coefficient the gain of all max_it sweeps [nd] and the decay of the last update
+  // whose norm the stop test reads [nd]; the bounds that certify it
+  const double *eig;
+  double eig_sum, eig_min;
   // mixed precision: the momentum inverse mass of the unit cell, [nd][nd] row-major
   // (M^-1 = K / area on an affine cell)
   const float *kinv;

@@ -35,6 +35,56 @@ static int bad_argument(const char *fn)
 
 namespace {
 
+// eigenvalues and vectors of the 1-D lumped-preconditioned mass D1^-1 M1: the symmetric
+// D1^-1/2 M1 D1^-1/2 = Q diag(lambda) Q^T by Jacobi rotations, Ve = D1^-1/2 Q and
+// Ved = Ve^-1 D1^-1 = Q^T D1^-1/2
+void eigen_1d(DegreeTables &t, int n1, double *lambda)
+{
+  double S[MAXN1][MAXN1], Q[MAXN1][MAXN1];
+  for (int i = 0; i < n1; ++i)
+    for (int j = 0; j < n1; ++j)
+      {
+        S[i][j] = t.M1[i][j] / std::sqrt(t.lumped[i] * t.lumped[j]);
+        Q[i][j] = i == j;
+      }
+  for (int sweep = 0; sweep < 30; ++sweep)
+    for (int i = 0; i < n1; ++i)
+      for (int j = i + 1; j < n1; ++j)
+        {
+          if (std::fabs(S[i][j]) < 1e-300)
+            continue;
+          const double th = 0.5 * std::atan2(2.0 * S[i][j], S[j][j] - S[i][i]);
+          const double c = std::cos(th), s = std::sin(th);
+          for (int k = 0; k < n1; ++k)
+            {
+              const double a = S[k][i], b = S[k][j];
+              S[k][i] = c * a - s * b;
+              S[k][j] = s * a + c * b;
+            }
+          for (int k = 0; k < n1; ++k)
+            {
+              const double a = S[i][k], b = S[j][k];
+              S[i][k] = c * a - s * b;
+              S[j][k] = s * a + c * b;
+            }
+          for (int k = 0; k < n1; ++k)
+            {
+              const double a = Q[k][i], b = Q[k][j];
+              Q[k][i] = c * a - s * b;
+              Q[k][j] = s * a + c * b;
+            }
+        }
+  for (int a = 0; a < n1; ++a)
+    {
+      lambda[a] = S[a][a];
+      for (int i = 0; i < n1; ++i)
+        {
+          t.Ve[i][a] = Q[i][a] / std::sqrt(t.lumped[i]);
+          t.Ved[a][i] = Q[i][a] / std::sqrt(t.lumped[i]);
+        }
+    }
+}
+
 DegreeTables make_tables(int p)
 {
   DegreeTables t;
@@ -99,7 +149,55 @@ DegreeTables make_tables(int p)
     for (int i = 0; i < n1; ++i)
       smax = std::max(smax, std::fabs(t.Sg[a][i]));
   t.lam = smax * smax;
+  double lambda[MAXN1];
+  eigen_1d(t, n1, lambda);
   return t;
+}
+
+// The capped sweeps of a wet cell in the eigenbasis (wet_depth_solve): with r the right-hand
+// side, c = (Ved x Ved) r / area, and mu = 1 - el_a el_b in [0, 1), update k (k = 1, 2, ..) is
+// (Ve x Ve) mu^(k-1) c, so K sweeps add up to (Ve x Ve) gain c with gain = sum_{k<K} mu^k.
+//   tab        gain [nd], then mu^(K-2) [nd] (1 for K < 3)
+//   sum_bound  sum_m gain_m |c_m| times this bounds the l1 norms of all updates together
+//   min_bound  the stop test |update|_1 <= 1e-12 cannot end the iteration before sweep K
+//              while max_m mu_m^(K-2) |c_m| exceeds this (an l1 norm is at least any
+//              eigen-coefficient over the largest entry of Ve^-1 x Ve^-1; mu <= 1)
+void sweep_tables(int p, int K, std::vector<double> &tab, double &sum_bound, double &min_bound)
+{
+  DegreeTables t = make_tables(p);
+  const int n1 = p + 1, nd = n1 * n1;
+  double lambda[MAXN1];
+  eigen_1d(t, n1, lambda);
+  tab.assign(2 * (size_t)nd, 0.0);
+  for (int b = 0; b < n1; ++b)
+    for (int a = 0; a < n1; ++a)
+      {
+        const double mu = std::max(0.0, 1.0 - lambda[a] * lambda[b]);
+        double gain = 0.0, pw = 1.0, last = 1.0;
+        for (int k = 0; k < K; ++k)
+          {
+            gain += pw;
+            if (k == K - 2)
+              last = pw;
+            pw *= mu;
+          }
+        tab[a + n1 * b] = gain;
+        tab[nd + a + n1 * b] = last;
+      }
+  double col = 0.0, inv = 0.0;
+  for (int a = 0; a < n1; ++a)
+    {
+      double s = 0.0;
+      for (int i = 0; i < n1; ++i)
+        {
+          s += std::fabs(t.Ve[i][a]);
+          inv = std::max(inv, std::fabs(t.Ved[a][i]) * t.lumped[i]);
+        }
+      col = std::max(col, s);
+    }
+  // a margin of 2 for rounding
+  sum_bound = 2.0 * col * col;
+  min_bound = K < 2 ? -1.0 : 2.0 * 1e-12 * inv * inv;
 }
 
 Basis<float> to_float(const DegreeTables &t)
@@ -423,6 +521,7 @@ void free_all(oc_dg *op)
   f(op->d_bz);
   f(op->d_btable);
   f(op->d_sweeps_blk);
+  f(op->d_eig);
   f(op->d_jmat);
   f(op->d_kinv);
   f(op->d_defer);
@@ -825,7 +924,9 @@ int oc_dg_create(const oc_mesh_desc *mesh, const oc_params *prm, oc_dg **out)
       delete op;
       return rc;
     }
-  if ((rc = upload(&op->d_hxy, hxy)) || (rc = upload(&op->d_order, op->order)) ||
+  std::vector<double> eig;
+  sweep_tables(op->P, op->max_it, eig, op->eig_sum, op->eig_min);
+  if ((rc = upload(&op->d_eig, eig)) || (rc = upload(&op->d_hxy, hxy)) || (rc = upload(&op->d_order, op->order)) ||
       (rc = upload(&op->d_nbr, nbr)) ||
       (rc = upload(&op->d_fid, fid)) || (rc = upload(&op->d_finfo, finfo)) ||
       (rc = upload(&op->d_bkind, bkind)) || (rc = dalloc(&op->d_sweeps_blk, (size_t)NB)) ||

@@ -1395,6 +1395,64 @@ __device__ __forceinline__ int depth_mass(const OpArgs &O, const DegreeTables &T
   return ndry;
 }
 
+// Z += Dinv R; returns the update's l1 norm.  R is advanced to the new Z by the linear
+// formula R <- R - area (M1 x M1) dZ (the next residual while the depth is linear in Z)
+template <int P, typename DinvFn>
+__device__ __forceinline__ double jacobi_update(const DegreeTables &T, double area, double *R,
+                                                double *Z, DinvFn dinv)
+{
+  constexpr int N1 = P + 1, ND = N1 * N1;
+  double dZ[ND], norm = 0.0;
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    {
+      const double old = Z[i];
+      Z[i] += dinv(i) * R[i];
+      dZ[i] = Z[i] - old;
+      norm += fabs(dZ[i]);
+    }
+#pragma unroll
+  for (int l = 0; l < N1; ++l)
+    {
+      double x[N1];
+#pragma unroll
+      for (int i = 0; i < N1; ++i)
+        {
+          double s = 0;
+#pragma unroll
+          for (int m = 0; m < N1; ++m)
+            s += T.M1[i][m] * dZ[m + N1 * l];
+          x[i] = s;
+        }
+#pragma unroll
+      for (int i = 0; i < N1; ++i)
+        dZ[i + N1 * l] = x[i];  // dZ now holds (M1 x I) dZ
+    }
+#pragma unroll
+  for (int j = 0; j < N1; ++j)
+#pragma unroll
+    for (int i = 0; i < N1; ++i)
+      {
+        double s = 0;
+#pragma unroll
+        for (int l = 0; l < N1; ++l)
+          s += T.M1[j][l] * dZ[i + N1 * l];
+        R[i + N1 * j] -= area * s;
+      }
+  return norm;
+}
+
+// one sweep of a cell that is wet at every GL point, with the full lumped mass
+template <int P>
+__device__ __forceinline__ double linear_sweep(const DegreeTables &T, double area,
+                                               double inv_area, double *R, double *Z)
+{
+  constexpr int N1 = P + 1;
+  return jacobi_update<P>(T, area, R, Z, [&](int i) {
+    return T.ilumped2[i % N1][i / N1] * inv_area;
+  });
+}
+
 // Jacobi solve of one cell: Z holds zeta^n on entry (and the dry lift is applied to it),
 // F the front; returns the number of sweeps.  OceanDG.h:1374-1507.
 template <int P>
@@ -1456,49 +1514,7 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
   double norm = 1.0, hbase = -1.0, C = 0.0;
   bool linear = false;
   double Rr[ND];
-  // Z += Dinv Rr and its l1 norm; the residual is advanced to the new Z by the linear
-  // formula (used only if the next sweep is certified linear, recomputed otherwise)
-  auto update = [&](auto dinv) {
-    norm = 0.0;
-    double dZ[ND];
-#pragma unroll
-    for (int i = 0; i < ND; ++i)
-      {
-        const double old = Z[i];
-        Z[i] += dinv(i) * Rr[i];
-        dZ[i] = Z[i] - old;
-        norm += fabs(dZ[i]);
-      }
-    C += norm;
-#pragma unroll
-    for (int l = 0; l < N1; ++l)
-      {
-        double x[N1];
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          {
-            double s = 0;
-#pragma unroll
-            for (int m = 0; m < N1; ++m)
-              s += T.M1[i][m] * dZ[m + N1 * l];
-            x[i] = s;
-          }
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          dZ[i + N1 * l] = x[i];  // dZ now holds (M1 x I) dZ
-      }
-#pragma unroll
-    for (int j = 0; j < N1; ++j)
-#pragma unroll
-      for (int i = 0; i < N1; ++i)
-        {
-          double s = 0;
-#pragma unroll
-          for (int l = 0; l < N1; ++l)
-            s += T.M1[j][l] * dZ[i + N1 * l];
-          Rr[i + N1 * j] -= area * s;
-        }
-  };
+  auto update = [&](auto dinv) { C += norm = jacobi_update<P>(T, area, Rr, Z, dinv); };
   auto wet_dinv = [&](int i) { return T.ilumped2[i % N1][i / N1] * inv_area; };
   int k = 0;
   for (; k < O.max_it && norm > 1e-12; ++k)
@@ -1558,6 +1574,144 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
         }
     }
   return k;
+}
+
+// FP64 depth solve of one cell: Z holds zeta^n on entry, r = sum_j a_j L_zeta,j; returns the
+// number of sweeps.  `front` (may be null): receives r + M h(zeta^n), entry i at i * CB.
+//
+// A cell that stays wet through the whole iteration (hmin, the least depth of zeta^n at the
+// GL points, exceeds what all updates together can take away) iterates a linear map on the
+// exact tensor-product mass: the first residual is r itself (the two depth integrals of the
+// front and of the residual cancel) and the capped sweeps have a closed form in the
+// eigenbasis of D^-1 M (sweep_tables), four 1-D contractions in all instead of two passes
+// over the GL points with their test-function integrals and up to max_it sweeps of two
+// contractions each.  Where the stop test could end the sweeps early (updates near 1e-12) the
+// linear sweeps run one by one, so that the count and the last update are the iteration's.
+// Every other cell takes jacobi_solve.  The solve is VALU work on the height wave's serial
+// chain, at p = 3 about 3700 instructions a cell before and 600 in closed form: an RK4 step
+// of 12,800 cells at p = 1 (latency-bound) 51.7 -> 40.3 us, of 2,500 at p = 2 124 -> 101 us,
+// of 97,280 at p = 3 (issue-bound) 407 -> 379 us.
+template <int P>
+__device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &T,
+                                           const Phys<double> &M, int batch, int lane,
+                                           double area, double *r, double *Z, double *front)
+{
+  constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
+  if (front)
+    {
+      double F[ND];
+#pragma unroll
+      for (int i = 0; i < ND; ++i)
+        F[i] = r[i];
+      unsigned long long bits = 0;
+      double hdummy;
+      depth_mass<P, false>(O, T, M, batch, lane, Z, F, 1.0, area, bits, hdummy);
+#pragma unroll
+      for (int i = 0; i < ND; ++i)
+        front[(size_t)i * CB] = F[i];
+    }
+  double hmin = DBL_MAX;
+  {
+    const size_t zbase = (size_t)batch * NG * NG * CB + lane;
+    const FieldV<double> bed = in_vgprs<double>(O.cell1);
+#pragma unroll 1
+    for (int b = 0; b < NG; ++b)
+      {
+        double zs[N1];
+#pragma unroll
+        for (int i = 0; i < N1; ++i)
+          {
+            double s = 0;
+#pragma unroll
+            for (int j = 0; j < N1; ++j)
+              s += T.Sg[b][j] * Z[i + N1 * j];
+            zs[i] = s;
+          }
+#pragma unroll
+        for (int a = 0; a < NG; ++a)
+          {
+            double z = 0;
+#pragma unroll
+            for (int i = 0; i < N1; ++i)
+              z += T.Sg[a][i] * zs[i];
+            hmin = fmin(hmin, z + fld(bed, zbase + (size_t)(a + NG * b) * CB));
+          }
+      }
+  }
+  // fmin drops NaN: a cell with a value that is not finite goes to jacobi_solve
+  double zsum = 0.0;
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    zsum += Z[i];
+  const double inv_area = 1.0 / area;
+  double c[ND], sum = 0.0, last = 0.0;
+  {
+    double X[ND];
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int a = 0; a < N1; ++a)
+        {
+          double s = 0;
+#pragma unroll
+          for (int i = 0; i < N1; ++i)
+            s += T.Ved[a][i] * r[i + N1 * j];
+          X[a + N1 * j] = s;
+        }
+#pragma unroll
+    for (int b = 0; b < N1; ++b)
+#pragma unroll
+      for (int a = 0; a < N1; ++a)
+        {
+          double s = 0;
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+            s += T.Ved[b][j] * X[a + N1 * j];
+          last = fmax(last, fabs(s) * O.eig[ND + a + N1 * b]);
+          c[a + N1 * b] = s * O.eig[a + N1 * b];
+          sum += fabs(c[a + N1 * b]);
+        }
+  }
+  if (hmin - T.lam * O.eig_sum * (sum * inv_area) > 2e-12 && zsum - zsum == 0.0)
+    {
+      if (last * inv_area > O.eig_min)
+        {
+          double X[ND];
+#pragma unroll
+          for (int b = 0; b < N1; ++b)
+#pragma unroll
+            for (int i = 0; i < N1; ++i)
+              {
+                double s = 0;
+#pragma unroll
+                for (int a = 0; a < N1; ++a)
+                  s += T.Ve[i][a] * c[a + N1 * b];
+                X[i + N1 * b] = s;
+              }
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i)
+              {
+                double s = 0;
+#pragma unroll
+                for (int b = 0; b < N1; ++b)
+                  s += T.Ve[j][b] * X[i + N1 * b];
+                Z[i + N1 * j] += s * inv_area;
+              }
+          return O.max_it;
+        }
+      int k = 0;
+      double norm = 1.0;
+#pragma unroll 1
+      for (; k < O.max_it && norm > 1e-12; ++k)
+        norm = linear_sweep<P>(T, area, inv_area, r, Z);
+      return k;
+    }
+  unsigned long long bits = 0;
+  double hdummy;
+  depth_mass<P, false>(O, T, M, batch, lane, Z, r, 1.0, area, bits, hdummy);
+  return jacobi_solve<P>(O, T, M, batch, lane, area, r, Z);
 }
 
 // Mixed precision depth solve.  When the cell is wet at every GL point with a margin the
@@ -1754,16 +1908,8 @@ __global__ __launch_bounds__(CB) void k_height_jacobi(OpArgs O, StageArgs S)
         k = mixed_depth_solve<P, false>(O, T, M, batch, lane, area, F, Z,
                                         have_jr ? jr : nullptr);
       else
-        {
-          unsigned long long bits = 0;
-          double hdummy;
-          depth_mass<P, false>(O, T, M, batch, lane, Z, F, 1.0, area, bits, hdummy);
-          if (S.scratch)
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              S.scratch[vix(batch, 1, 0, ND, i, lane)] = F[i];
-          k = jacobi_solve<P>(O, T, M, batch, lane, area, F, Z);
-        }
+        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z,
+                           S.scratch ? S.scratch + (size_t)batch * ND * CB + lane : nullptr);
 #pragma unroll
       for (int i = 0; i < ND; ++i)
         S.rk_dst[vix(batch, 1, 0, ND, i, lane)] = Z[i];
@@ -1969,16 +2115,8 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
         k = mixed_depth_solve<P, defer_depth_solve(P)>(O, T, M, batch, lane, area, F, Z,
                                                        have_jr ? jr : nullptr);
       else
-        {
-          unsigned long long bits = 0;
-          double hdummy;
-          depth_mass<P, false>(O, T, M, batch, lane, Z, F, 1.0, area, bits, hdummy);
-          if (S.scratch)
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              S.scratch[vix(batch, 1, 0, ND, i, lane)] = F[i];
-          k = jacobi_solve<P>(O, T, M, batch, lane, area, F, Z);
-        }
+        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z,
+                           S.scratch ? S.scratch + (size_t)batch * ND * CB + lane : nullptr);
       if (centred<R>() && S.out32)
         {
           // the next stage input in its centred FP32 form: zeta minus its DoF-0 value, and
