@@ -88,8 +88,7 @@ __device__ __forceinline__ void stiff_source(const OpArgs &O, const Basis<R> &T,
           const R h = M.depth(z, zb);
           const R s = M.inv_depth(h);
           const R vx = qx * s, vy = qy * s;
-          const R inv_d = R(1) / (exp(log(h) * R(0.33333333333)));
-          const R hcf = M.g * n_m * n_m * inv_d * sqrt(vx * vx + vy * vy);
+          const R hcf = manning_coefficient(M.g, n_m, h, vx, vy);
           const R JxW = T.wq[a] * T.wq[b] * area;
           const R v0 = -(hcf * vx) * JxW, v1 = -(hcf * vy) * JxW;
 #pragma unroll
@@ -252,8 +251,8 @@ __device__ __forceinline__ void ark_update_cell(const OpArgs &O, const ArkArgs &
           const double s = M.inv_depth(h);
           const double vx = qx[k] * s, vy = qy[k] * s;
           // BottomFrictionManning::jacobian (BottomFriction.h:201-212)
-          const double jac = M.g * cf * cf * (1. / (exp(log(h) * 1.33333333333))) *
-                             sqrt(vx * vx + vy * vy);
+          const double jac = M.g * cf * cf * ManningPowers(h).four_thirds() *
+                             sqrt_nr(vx * vx + vy * vy);
           iw[k] *= 1. / (1. + A.fm * jac);
         }
     }

@@ -1033,8 +1033,7 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
           if (O.has_friction)
             {
               const R n_m = R(fld(O.cell0[1], pi));
-              const R inv_d = R(1) / (exp(log(h) * R(0.33333333333)));
-              const R hcf = g * n_m * n_m * inv_d * sqrt(vx * vx + vy * vy);
+              const R hcf = manning_coefficient(g, n_m, h, vx, vy);
               Sx -= hcf * vx;
               Sy -= hcf * vy;
             }
