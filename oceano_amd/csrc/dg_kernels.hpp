@@ -41,6 +41,7 @@ struct Basis
   // 1-D eigenvectors of D1^-1 M1 (D1 the lumped mass): M1 = D1 Ve diag(el) Ved, with Ved =
   // Ve^-1 D1^-1, so that (Ved x Ved) r are the eigen-coefficients of D^-1 r on the unit cell
   R Ve[MAXN1][MAXN1], Ved[MAXN1][MAXN1];
+  R Kn[MAXN1][MAXN1];  // 1-D inverse mass of the unit interval: sum_a Ti[i][a] Ti[j][a] / wn[a]
   R lam;                     // max_{a,i} Sg[a][i]^2: bound of |phi_ij| at the GL(ng)^2 points
 };
 using DegreeTables = Basis<double>;

@@ -129,6 +129,10 @@ DegreeTables make_tables(int p)
     for (int a = 0; a < n1; ++a)
       t.Ti[i][a] = Si[i * n1 + a];
   for (int i = 0; i < n1; ++i)
+    for (int j = 0; j < n1; ++j)
+      for (int a = 0; a < n1; ++a)
+        t.Kn[i][j] += t.Ti[i][a] * t.Ti[j][a] / t.wn[a];
+  for (int i = 0; i < n1; ++i)
     {
       double s = 0;
       for (int a = 0; a < ng; ++a)
@@ -256,22 +260,17 @@ std::vector<float> jacobi_matrix(int p, int K)
 
 // The momentum inverse mass of the unit cell as one matrix: the basis change of
 // CellwiseInverseMassMatrix (OceanDG.h:1541-1553) from GL(p+1) nodal values to Gauss(p+1)
-// collocation, the inverse quadrature weights and back, is B1 (x) B1 with
-// B1[i][j] = sum_a Ti[i][a] Ti[j][a] / wn[a]; on a cell of area |K|, M^-1 = (B1 (x) B1) / |K|.
+// collocation, the inverse quadrature weights and back, is Kn (x) Kn (Basis::Kn); on a cell of
+// area |K|, M^-1 = (Kn (x) Kn) / |K|.
 // Row-major [nd][nd], node index i + n1 j (x fastest).
 std::vector<float> inverse_mass_matrix(int p)
 {
   const DegreeTables t = make_tables(p);
   const int n1 = p + 1, nd = n1 * n1;
-  std::vector<double> B(n1 * n1, 0.0);
-  for (int i = 0; i < n1; ++i)
-    for (int j = 0; j < n1; ++j)
-      for (int a = 0; a < n1; ++a)
-        B[i * n1 + j] += t.Ti[i][a] * t.Ti[j][a] / t.wn[a];
   std::vector<float> out(nd * nd);
   for (int r = 0; r < nd; ++r)
     for (int c = 0; c < nd; ++c)
-      out[r * nd + c] = float(B[(r % n1) * n1 + (c % n1)] * B[(r / n1) * n1 + (c / n1)]);
+      out[r * nd + c] = float(t.Kn[r % n1][c % n1] * t.Kn[r / n1][c / n1]);
   return out;
 }
 
