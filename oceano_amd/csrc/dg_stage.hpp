@@ -902,7 +902,7 @@ constexpr int discharge_lds_words()
 // touches only the cell's N1 DoFs on that face, so the swap moves 4 N1 momentum values
 // (ROLE 0 -> 1) and 2 N1 mass values (ROLE 1 -> 0) per cell through `xch`
 // (pair_xch_words() words of LDS).  Both waves call it once, every lane (one workgroup
-// barrier).
+// barrier); `meanwhile` runs between a wave's hand-over and the barrier.
 // ---------------------------------------------------------------------------------------
 template <int P>
 __host__ __device__ constexpr int pair_xch_words()
@@ -910,8 +910,9 @@ __host__ __device__ constexpr int pair_xch_words()
   return 6 * (P + 1) * CB;
 }
 
-template <int P, typename R, int ROLE>
-__device__ __forceinline__ void pair_exchange(R (&A)[3][(P + 1) * (P + 1)], R *xch)
+template <int P, typename R, int ROLE, typename Fn>
+__device__ __forceinline__ void pair_exchange(R (&A)[3][(P + 1) * (P + 1)], R *xch,
+                                              Fn meanwhile)
 {
   constexpr int N1 = P + 1;
   const int lane = threadIdx.x & (CB - 1);
@@ -935,6 +936,7 @@ __device__ __forceinline__ void pair_exchange(R (&A)[3][(P + 1) * (P + 1)], R *x
         for (int k = 0; k < N1; ++k)
           xch[(4 * N1 + (f - 2) * N1 + k) * CB + lane] = A[0][face_dof<N1>(f, k)];
     }
+  meanwhile();
   __syncthreads();
   if constexpr (ROLE == 0)
     {
@@ -1234,7 +1236,7 @@ __device__ __forceinline__ void discharge_block(const OpArgs &O, const StageArgs
           face_terms<P, 3, R, 0xC>(O, T, batch, lane, hx, hy, Z, QX, QY, zc, src_h, src_q, A,
                                    fn, fn, IN32);
         }
-      pair_exchange<P, R, 1>(A, xch);
+      pair_exchange<P, R, 1>(A, xch, [] {});
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -1610,11 +1612,50 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
   return k;
 }
 
+// least depth of zeta^n = Z at the GL(p+2) points; NaN where an entry of Z is not finite (fmin
+// drops NaN), which no cell's certificate passes
+template <int P>
+__device__ __forceinline__ double least_depth(const OpArgs &O, const DegreeTables &T, int batch,
+                                              int lane, const double *Z)
+{
+  constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
+  double hmin = DBL_MAX;
+  const size_t zbase = (size_t)batch * NG * NG * CB + lane;
+  const FieldV<double> bed = in_vgprs<double>(O.cell1);
+#pragma unroll 1
+  for (int b = 0; b < NG; ++b)
+    {
+      double zs[N1];
+#pragma unroll
+      for (int i = 0; i < N1; ++i)
+        {
+          double s = 0;
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+            s += T.Sg[b][j] * Z[i + N1 * j];
+          zs[i] = s;
+        }
+#pragma unroll
+      for (int a = 0; a < NG; ++a)
+        {
+          double z = 0;
+#pragma unroll
+          for (int i = 0; i < N1; ++i)
+            z += T.Sg[a][i] * zs[i];
+          hmin = fmin(hmin, z + fld(bed, zbase + (size_t)(a + NG * b) * CB));
+        }
+    }
+  double zsum = 0.0;
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    zsum += Z[i];
+  return hmin + (zsum - zsum);
+}
+
 // FP64 depth solve of one cell: Z holds zeta^n on entry, r = sum_j a_j L_zeta,j; returns the
 // number of sweeps.  `front` (may be null): receives r + M h(zeta^n), entry i at i * CB.
 //
-// A cell that stays wet through the whole iteration (hmin, the least depth of zeta^n at the
-// GL points, exceeds what all updates together can take away) iterates a linear map on the
+// A cell that stays wet through the whole iteration (hmin = least_depth exceeds what all updates together can take away) iterates a linear map on the
 // exact tensor-product mass: the first residual is r itself (the two depth integrals of the
 // front and of the residual cancel) and the capped sweeps have a closed form in the
 // eigenbasis of D^-1 M (sweep_tables), four 1-D contractions in all instead of two passes
@@ -1628,9 +1669,10 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
 template <int P>
 __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &T,
                                            const Phys<double> &M, int batch, int lane,
-                                           double area, double *r, double *Z, double *front)
+                                           double area, double *r, double *Z, double hmin,
+                                           double *front)
 {
-  constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
+  constexpr int N1 = P + 1, ND = N1 * N1;
   if (front)
     {
       double F[ND];
@@ -1644,39 +1686,6 @@ __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &
       for (int i = 0; i < ND; ++i)
         front[(size_t)i * CB] = F[i];
     }
-  double hmin = DBL_MAX;
-  {
-    const size_t zbase = (size_t)batch * NG * NG * CB + lane;
-    const FieldV<double> bed = in_vgprs<double>(O.cell1);
-#pragma unroll 1
-    for (int b = 0; b < NG; ++b)
-      {
-        double zs[N1];
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          {
-            double s = 0;
-#pragma unroll
-            for (int j = 0; j < N1; ++j)
-              s += T.Sg[b][j] * Z[i + N1 * j];
-            zs[i] = s;
-          }
-#pragma unroll
-        for (int a = 0; a < NG; ++a)
-          {
-            double z = 0;
-#pragma unroll
-            for (int i = 0; i < N1; ++i)
-              z += T.Sg[a][i] * zs[i];
-            hmin = fmin(hmin, z + fld(bed, zbase + (size_t)(a + NG * b) * CB));
-          }
-      }
-  }
-  // fmin drops NaN: a cell with a value that is not finite goes to jacobi_solve
-  double zsum = 0.0;
-#pragma unroll
-  for (int i = 0; i < ND; ++i)
-    zsum += Z[i];
   const double inv_area = 1.0 / area;
   double c[ND], sum = 0.0, last = 0.0;
   {
@@ -1706,7 +1715,7 @@ __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &
           sum += fabs(c[a + N1 * b]);
         }
   }
-  if (hmin - T.lam * O.eig_sum * (sum * inv_area) > 2e-12 && zsum - zsum == 0.0)
+  if (hmin - T.lam * O.eig_sum * (sum * inv_area) > 2e-12)
     {
       if (last * inv_area > O.eig_min)
         {
@@ -1746,6 +1755,49 @@ __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &
   double hdummy;
   depth_mass<P, false>(O, T, M, batch, lane, Z, r, 1.0, area, bits, hdummy);
   return jacobi_solve<P>(O, T, M, batch, lane, area, r, Z);
+}
+
+// the same for the FP32 stage: formed in FP32 on the deviation from node 0
+template <int P>
+__device__ __forceinline__ float least_depth32(const OpArgs &O, int batch, int lane,
+                                               const double *Z)
+{
+  constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
+  const Basis<float> &Tf = basis<float>(P);
+  const double zc = Z[0];
+  float dev[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    dev[i] = float(Z[i] - zc);
+  float hmin = FLT_MAX;
+  const size_t zbase = (size_t)batch * NG * NG * CB + lane;
+  const FieldV<double> bed = in_vgprs<double>(O.cell1);
+#pragma unroll 1
+  for (int b = 0; b < NG; ++b)
+    {
+      float zs[N1];
+#pragma unroll
+      for (int i = 0; i < N1; ++i)
+        {
+          float s = 0;
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+            s += Tf.Sg[b][j] * dev[i + N1 * j];
+          zs[i] = s;
+        }
+#pragma unroll
+      for (int a = 0; a < NG; ++a)
+        {
+          float z = 0;
+#pragma unroll
+          for (int i = 0; i < N1; ++i)
+            z += Tf.Sg[a][i] * zs[i];
+          const double zb = fld(bed, zbase + (size_t)(a + NG * b) * CB);
+          const float h = float(zc + zb) + z;
+          hmin = h < hmin ? h : hmin;
+        }
+    }
+  return hmin;
 }
 
 // Mixed precision depth solve.  When the cell is wet at every GL point with a margin the
@@ -1794,44 +1846,9 @@ template <int P, bool DEFER>
 __device__ __forceinline__ int mixed_depth_solve(const OpArgs &O, const DegreeTables &T,
                                                  const Phys<double> &M, int batch, int lane,
                                                  double area, const double *r, double *Z,
-                                                 const float *jr)
+                                                 float hmin, const float *jr)
 {
-  constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
-  const Basis<float> &Tf = basis<float>(P);
-  // minimum depth of zeta^n over the GL points (FP32 on the deviation from node 0)
-  const double zc = Z[0];
-  float dev[ND];
-#pragma unroll
-  for (int i = 0; i < ND; ++i)
-    dev[i] = float(Z[i] - zc);
-  float hmin = FLT_MAX;
-  const size_t zbase = (size_t)batch * NG * NG * CB + lane;
-  const FieldV<double> bed = in_vgprs<double>(O.cell1);
-#pragma unroll 1
-  for (int b = 0; b < NG; ++b)
-    {
-      float zs[N1];
-#pragma unroll
-      for (int i = 0; i < N1; ++i)
-        {
-          float s = 0;
-#pragma unroll
-          for (int j = 0; j < N1; ++j)
-            s += Tf.Sg[b][j] * dev[i + N1 * j];
-          zs[i] = s;
-        }
-#pragma unroll
-      for (int a = 0; a < NG; ++a)
-        {
-          float z = 0;
-#pragma unroll
-          for (int i = 0; i < N1; ++i)
-            z += Tf.Sg[a][i] * zs[i];
-          const double zb = fld(bed, zbase + (size_t)(a + NG * b) * CB);
-          const float h = float(zc + zb) + z;
-          hmin = h < hmin ? h : hmin;
-        }
-    }
+  constexpr int ND = (P + 1) * (P + 1);
   float rf[1][ND];
 #pragma unroll
   for (int i = 0; i < ND; ++i)
@@ -1940,9 +1957,10 @@ __global__ __launch_bounds__(CB) void k_height_jacobi(OpArgs O, StageArgs S)
     {
       if (centred<R>())
         k = mixed_depth_solve<P, false>(O, T, M, batch, lane, area, F, Z,
+                                        least_depth32<P>(O, batch, lane, Z),
                                         have_jr ? jr : nullptr);
       else
-        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z,
+        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z, least_depth<P>(O, T, batch, lane, Z),
                            S.scratch ? S.scratch + (size_t)batch * ND * CB + lane : nullptr);
 #pragma unroll
       for (int i = 0; i < ND; ++i)
@@ -2044,7 +2062,50 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
   const Phys<double> M = physics<double>(O);
   int k = 0;
   double F[ND], Z[ND], area = 1.0;
+  typename std::conditional<centred<R>(), float, double>::type hmin = 0;
   R Racc[1][ND];
+  // what the front and the solve need besides this stage's L_zeta: the earlier k vectors'
+  // part of the front, summed in the reference's order (one whole vector at a time, its loads
+  // in flight together); zeta^n and its least depth
+  auto prepare_front = [&] {
+    if (!active || S.stage == 0)
+      return;
+    const size_t base = (size_t)batch * ND * CB + lane;
+    const R *k0 = reinterpret_cast<const R *>(S.kprev[0]) + base;
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      F[i] = double(k0[(size_t)i * CB]);
+    issue_barrier();
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      F[i] = S.factor[0] * F[i];
+    for (int j = 1; j < S.stage; ++j)
+      {
+        const R *kp = reinterpret_cast<const R *>(S.kprev[j]) + base;
+        const double fj = S.factor[j];
+        double t[ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          t[i] = double(kp[(size_t)i * CB]);
+        issue_barrier();
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          F[i] += fj * t[i];
+      }
+  };
+  auto prepare_depth = [&] {
+    if (!active)
+      return;
+    phase_barrier();
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      Z[i] = S.wsol[vix(batch, 1, 0, ND, i, lane)];
+    issue_barrier();
+    if constexpr (centred<R>())
+      hmin = least_depth32<P>(O, batch, lane, Z);
+    else
+      hmin = least_depth<P>(O, T, batch, lane, Z);
+  };
   if constexpr (PAIR)
     {
       // faces 0 and 1 for both equations; the momentum integrals go to the discharge wave,
@@ -2073,7 +2134,18 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
           face_terms<P, 3, R, 0x3>(O, basis<R>(P), batch, lane, R(hx), R(hy), Zo, QX, QY, zc,
                                    S.src_h, S.src_q, A, fn, fn, IN32);
         }
-      pair_exchange<P, R, 0>(A, xch);
+      // at p >= 2 the height wave reaches the exchange first (p = 3, 97,280 cells: 17 us into the
+      // workgroup against 26 in FP64, 19 against 25 in mixed precision) and waits: it prepares
+      // the solve before the barrier.  RK4 step FP64 375 -> 359 us, mixed 179 -> 177; 2,500
+      // cells at p = 2, FP64 83 -> 79 us.  At p = 1 both waves arrive together and it would
+      // only delay the other (819,200 cells, mixed: 300 -> 302 us)
+      pair_exchange<P, R, 0>(A, xch, [&] {
+        if constexpr (P >= 2)
+          {
+            prepare_front();
+            prepare_depth();
+          }
+      });
 #pragma unroll
       for (int i = 0; i < ND; ++i)
         Racc[0][i] = A[0][i];
@@ -2089,56 +2161,29 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
                             (const R *)Zo, (const R *)QX, (const R *)QY, zc, S.src_h,
                             S.src_q, Racc);
     }
+  constexpr bool PREPARED = PAIR && P >= 2;
+  if (active)
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      reinterpret_cast<R *>(S.dst)[vix(batch, 1, 0, ND, i, lane)] = Racc[0][i];  // ki_h[stage+1]
+  if constexpr (!PREPARED)
+    prepare_front();
   if (active)
     {
-      {
-        // front sum_j a_j k_{j+1} in the reference's order, the earlier k vectors read one
-        // whole vector at a time (loads in flight together)
-        const size_t base = (size_t)batch * ND * CB + lane;
+      const double fs = S.factor[S.stage];
+      if (S.stage == 0)
+        {
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            F[i] = fs * double(Racc[0][i]);
+        }
+      else
 #pragma unroll
         for (int i = 0; i < ND; ++i)
-          reinterpret_cast<R *>(S.dst)[base + (size_t)i * CB] = Racc[0][i];  // ki_h[stage+1]
-        if (S.stage == 0)
-          {
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              F[i] = S.factor[0] * double(Racc[0][i]);
-          }
-        else
-          {
-            const R *k0 = reinterpret_cast<const R *>(S.kprev[0]) + base;
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              F[i] = double(k0[(size_t)i * CB]);
-            issue_barrier();
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              F[i] = S.factor[0] * F[i];
-            for (int j = 1; j < S.stage; ++j)
-              {
-                const R *kp = reinterpret_cast<const R *>(S.kprev[j]) + base;
-                const double fj = S.factor[j];
-                double t[ND];
-#pragma unroll
-                for (int i = 0; i < ND; ++i)
-                  t[i] = double(kp[(size_t)i * CB]);
-                issue_barrier();
-#pragma unroll
-                for (int i = 0; i < ND; ++i)
-                  F[i] += fj * t[i];
-              }
-            const double fs = S.factor[S.stage];
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-              F[i] += fs * double(Racc[0][i]);
-          }
-      }
-      phase_barrier();
-#pragma unroll
-      for (int i = 0; i < ND; ++i)
-        Z[i] = S.wsol[vix(batch, 1, 0, ND, i, lane)];
-      issue_barrier();
+          F[i] += fs * double(Racc[0][i]);
     }
+  if constexpr (!PREPARED)
+    prepare_depth();
   float jr[ND];
   bool have_jr = false;
   if constexpr (centred<R>())
@@ -2146,10 +2191,10 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
   if (active)
     {
       if (centred<R>())
-        k = mixed_depth_solve<P, defer_depth_solve(P)>(O, T, M, batch, lane, area, F, Z,
+        k = mixed_depth_solve<P, defer_depth_solve(P)>(O, T, M, batch, lane, area, F, Z, hmin,
                                                        have_jr ? jr : nullptr);
       else
-        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z,
+        k = depth_solve<P>(O, T, M, batch, lane, area, F, Z, hmin,
                            S.scratch ? S.scratch + (size_t)batch * ND * CB + lane : nullptr);
       if (centred<R>() && S.out32)
         {
