@@ -88,53 +88,100 @@ __global__ __launch_bounds__(CB) void k_closure_features(OpArgs O, ClosureArgs C
       C.features[row + i] = f[i];
 }
 
+// The correction of 16 cells per wave and pass.  The lanes are 16 cells x 4 groups: group g < 3
+// forms the modal coefficients of field g (zeta, hu, hv), group 3 takes the statistics; after
+// the network group g brings half of the nodes of component g / 2 back to nodal values.  A cell
+// gets tau = 0 unless it is active and all its outputs are finite.
+// Latency bounds it (2,500 cells are 157 waves): 16 cells per wave instead of 64 cells and four
+// tiles in turn, weights in registers (ForwardWeights): 33.0 -> 9.6 us.
 template <int P>
 __global__ __launch_bounds__(CB) void k_closure(OpArgs O, ClosureArgs C)
 {
   using namespace mlp;
-  constexpr int ND = (P + 1) * (P + 1);
-  __shared__ __attribute__((aligned(16))) bf16 s_wt[NT];
-  __shared__ __attribute__((aligned(16))) bf16 s_x[CB * IN];
-  __shared__ __attribute__((aligned(16))) bf16 s_h[3][16 * HID];
-  __shared__ float s_y[CB * OUT];
-  const int batch = logical_batch(blockIdx.x, O.n_batches, O.xcd_swizzle);
-  const int lane = threadIdx.x;
-  for (int i = lane; i < NT; i += CB)
-    s_wt[i] = C.wt[i];
-  const bool active = batch * CB + lane < O.n_cells;
-  float f[IN];
-  if (active)
-    closure_features<P>(C, batch, lane, f);
-#pragma unroll
-  for (int k = 0; k < IN; ++k)
+  constexpr int ND = (P + 1) * (P + 1), TILES = CB / 16;
+  static_assert(3 * ND + 3 <= IN && 2 * ND <= OUT, "closure network too narrow");
+  __shared__ __attribute__((aligned(16))) bf16 s_x[16 * IN];
+  __shared__ __attribute__((aligned(16))) bf16 s_h[2][16 * LDT];
+  __shared__ float s_y[16 * OUT];
+  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+  ForwardWeights W;
+  W.load(C.wt, C.p);
+  const int n_tiles = (O.n_cells + 15) / 16;
+  for (int tile = logical_batch(blockIdx.x, gridDim.x, O.xcd_swizzle); tile < n_tiles;
+       tile += gridDim.x)
     {
-      const float x = (active && k < C.n_in) ? (f[k] - C.norm[k]) * C.norm[IN + k] : 0.f;
-      s_x[lane * IN + k] = to_bf16(x);
+      const int batch = tile / TILES, cl = (tile % TILES) * 16 + r;
+      const bool inside = tile * 16 + r < O.n_cells;
+      if (g < 3)
+        {
+          const double *src = g == 0 ? C.zeta + vix(batch, 1, 0, ND, 0, cl)
+                                     : C.q + vix(batch, 2, g - 1, ND, 0, cl);
+          double u[ND];
+#pragma unroll
+          for (int k = 0; k < ND; ++k)
+            u[k] = inside ? src[k * CB] : 0.0;
+#pragma unroll
+          for (int m = 0; m < ND; ++m)
+            {
+              double a = 0;
+#pragma unroll
+              for (int k = 0; k < ND; ++k)
+                a += C.vi[m * ND + k] * u[k];
+              const int i = g * ND + m;
+              s_x[r * IN + i] =
+                to_bf16(inside ? (float(a) - C.norm[i]) * C.norm[IN + i] : 0.f);
+            }
+        }
+      else
+        {
+#pragma unroll
+          for (int i = 3 * ND; i < IN; ++i)
+            {
+              float x = 0.f;
+              if (i < 3 * ND + 3 && inside)
+                x = (float(C.stats[((size_t)batch * 4 + i - 3 * ND) * CB + cl]) - C.norm[i]) *
+                    C.norm[IN + i];
+              s_x[r * IN + i] = to_bf16(x);
+            }
+        }
+      tile_fence();
+      f32x4 out[OUT / 16];
+      forward_tile(load8(s_x + r * IN + 8 * g), W, s_h, out);
+#pragma unroll
+      for (int ct = 0; ct < OUT / 16; ++ct)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s_y[(4 * g + j) * OUT + 16 * ct + r] = out[ct][j];
+      tile_fence();
+      const int c = g >> 1;
+      double tm[ND];
+      bool finite = inside && C.stats[((size_t)batch * 4 + 3) * CB + cl] != 0.0;
+#pragma unroll
+      for (int m = 0; m < ND; ++m)
+        {
+          const float y = output_value(s_y[r * OUT + c * ND + m], C.norm, c * ND + m);
+          finite = finite && isfinite(y);
+          tm[m] = double(y);
+        }
+      // both components of the cell: groups 0 and 2
+      const unsigned long long ok = __ballot(finite);
+      finite = ((ok >> r) & (ok >> (r + 32)) & 1ull) != 0;
+      constexpr int HALF = (ND + 1) / 2;
+      const bool hi = g & 1;
+#pragma unroll
+      for (int i = 0; i < HALF; ++i)
+        {
+          constexpr int LAST = ND - 1;
+          const int k_hi = HALF + i <= LAST ? HALF + i : LAST;
+          double t = 0;
+#pragma unroll
+          for (int m = 0; m < ND; ++m)
+            t += (hi ? C.v[k_hi * ND + m] : C.v[i * ND + m]) * tm[m];
+          if (!hi || HALF + i <= LAST)
+            C.tau[vix(batch, 2, c, ND, hi ? k_hi : i, cl)] = finite ? t : 0.0;
+        }
+      tile_fence();
     }
-  __syncthreads();
-  for (int rt = 0; rt < CB / 16; ++rt)
-    forward_tile(s_x + rt * 16 * IN, s_wt, C.p, s_h[0], s_h[1], s_h[2], nullptr,
-                 s_y + rt * 16 * OUT);
-  double tm[2 * ND];
-  bool finite = active && C.stats[((size_t)batch * 4 + 3) * CB + lane] != 0.0;
-#pragma unroll
-  for (int o = 0; o < 2 * ND; ++o)
-    {
-      const float y = output_value(s_y[lane * OUT + o], C.norm, o);
-      finite = finite && isfinite(y);
-      tm[o] = double(y);
-    }
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int k = 0; k < ND; ++k)
-      {
-        double t = 0;
-#pragma unroll
-        for (int m = 0; m < ND; ++m)
-          t += C.v[k * ND + m] * tm[c * ND + m];
-        C.tau[vix(batch, 2, c, ND, k, lane)] = finite ? t : 0.0;
-      }
 }
 
 // features != nullptr: write the network inputs of every cell (k_closure_features);
@@ -167,7 +214,11 @@ int launch_closure(oc_dg *op, const OpArgs &O, const double *zeta, const double 
       else
         {
           oc_mlp_device_state(op->closure_mlp, &C.p, &C.wt, &C.norm);
-          hipLaunchKernelGGL((k_closure<P>), dim3(op->NB), dim3(CB), 0, s, O, C);
+          // a wave per 16 cells up to 4 waves per SIMD, then each wave keeps its weights for
+          // several tiles
+          const int tiles = (op->N + 15) / 16;
+          hipLaunchKernelGGL((k_closure<P>), dim3(tiles < 4096 ? tiles : 4096), dim3(CB), 0, s, O,
+                             C);
         }
       HIP_TRY(hipGetLastError());
       return OC_OK;

@@ -1,8 +1,8 @@
 // mlp.hip -- training and inference of the closure network (BF16 MFMA, FP32 accumulation).
 //
-// Training step = k_mlp_grad (forward of 16-sample tiles, MSE loss, backward; each block
-// accumulates its weight gradients in LDS and writes one partial) + k_mlp_reduce (sum of
-// the partials in block order: deterministic) + k_mlp_adam (Adam in FP32 on the master
+// Training step = k_mlp_grad (forward of 16-sample tiles, MSE loss, backward; each wave
+// accumulates its weight gradients in registers and writes one partial) + k_mlp_reduce (sum of
+// the partials in a fixed order: deterministic) + k_mlp_adam (Adam in FP32 on the master
 // parameters, then the BF16 copies the products read).
 #include <hip/hip_runtime.h>
 
@@ -46,217 +46,289 @@ namespace {
     }                                                                \
   while (0)
 
-constexpr int WB0 = W2, NWB = B4 - W2;  // backward weights W2..W4 (row-major, with bias gaps)
-
-__global__ __launch_bounds__(64) void k_mlp_grad(const float *__restrict__ p,
-                                                 const bf16 *__restrict__ wt_g,
-                                                 const bf16 *__restrict__ wb_g,
-                                                 const float *__restrict__ norm, int64_t n,
-                                                 int n_in, int n_out,
-                                                 const float *__restrict__ X,
-                                                 const float *__restrict__ T, float gscale,
-                                                 float *__restrict__ partial,
-                                                 float *__restrict__ lossp)
+// X rows base .. base + 15 as the A operand of a tile: row l % 16, inputs 8 (l / 16) .., normalised
+// (mu, is: the lane's 8 means and inverse spreads), zero outside the n rows and n_in inputs
+__device__ __forceinline__ bf16x8 load_inputs(const float *__restrict__ X, int64_t base, int64_t n,
+                                              int n_in, const float (&mu)[8],
+                                              const float (&is)[8])
 {
-  __shared__ __attribute__((aligned(16))) bf16 s_wt[NT];
-  __shared__ __attribute__((aligned(16))) bf16 s_wb[NWB];
-  __shared__ float s_g[NPARAM];
-  __shared__ __attribute__((aligned(16))) bf16 s_x[16 * IN];
-  __shared__ __attribute__((aligned(16))) bf16 s_h[3][16 * HID];
-  __shared__ float s_z[3 * 16 * HID];
-  __shared__ float s_y[16 * OUT], s_t[16 * OUT];
-  __shared__ __attribute__((aligned(16))) bf16 s_d[2][16 * HID];
-  __shared__ float s_df[2][16 * HID];
-  __shared__ float s_norm[NNORM];
-  __shared__ float s_loss[64];
-  const int l = threadIdx.x, r = l & 15, kq = (l >> 4) * 4, k8 = (l >> 4) * 8;
-  for (int i = l; i < NT; i += 64)
-    s_wt[i] = wt_g[i];
-  for (int i = l; i < NWB; i += 64)
-    s_wb[i] = wb_g[WB0 + i];
-  for (int i = l; i < NPARAM; i += 64)
-    s_g[i] = 0.f;
-  for (int i = l; i < NNORM; i += 64)
-    s_norm[i] = norm[i];
+  const int l = threadIdx.x & 63, k8 = (l >> 4) * 8;
+  const int64_t row = base + (l & 15);
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    v[j] = row < n && k8 + j < n_in ? X[row * n_in + k8 + j] : mu[j];
+  bf16 h[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    h[j] = to_bf16((v[j] - mu[j]) * is[j]);
+  bf16x8 x;
+  __builtin_memcpy(&x, h, sizeof(x));
+  return x;
+}
+
+// Forward, loss and gradient of the rows of chunks blockIdx.x, blockIdx.x + gridDim.x, ... of 16
+// samples; one wave per workgroup writes one partial gradient.
+//
+// The chain of one chunk (eight dependent products, three GELUs) bounds it, not its 150 MFMAs:
+// at 4096 rows every wave has one chunk.  So nothing waits in it that need not: the weights of both
+// directions and the weight gradients stay in registers (one wave per SIMD has 512), and an
+// accumulator's layout (sample 4 (l / 16) + j, unit 16 ct + l % 16) is already the operand
+// layout of the 16-sample weight-gradient products, so only the row operands of the layer
+// products cross LDS.  4096 rows: about 56 us with weights and gradients in LDS, 26.5 us.
+__global__ __launch_bounds__(64, 1) void k_mlp_grad(const float *__restrict__ p,
+                                                    const bf16 *__restrict__ wt,
+                                                    const bf16 *__restrict__ wb,
+                                                    const float *__restrict__ norm, int64_t n,
+                                                    int n_in, int n_out,
+                                                    const float *__restrict__ X,
+                                                    const float *__restrict__ T, float gscale,
+                                                    float *__restrict__ partial,
+                                                    float *__restrict__ lossp)
+{
+  constexpr int HT = HID / 16, OT = OUT / 16, IT = IN / 16;
+  __shared__ __attribute__((aligned(16))) bf16 s_h[2][16 * LDT];
+  const int l = threadIdx.x, r = l & 15, g = l >> 4, kq = g * 4, k8 = g * 8;
+  ForwardWeights W;
+  W.load(wt, p);
+  // B operands of the backward products dZ W^T: row-major W rows, 16 bytes each
+  bf16x8 v2[2 * HT], v3[2 * HT], v4[HT];
+#pragma unroll
+  for (int ct = 0; ct < HT; ++ct)
+    {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+        {
+          v2[2 * ct + kk] = load8(wb + W2 + (16 * ct + r) * HID + 32 * kk + k8);
+          v3[2 * ct + kk] = load8(wb + W3 + (16 * ct + r) * HID + 32 * kk + k8);
+        }
+      v4[ct] = load8(wb + W4 + (16 * ct + r) * OUT + k8);
+    }
+  float mu[8], is[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    {
+      mu[j] = norm[k8 + j];
+      is[j] = norm[IN + k8 + j];
+    }
+  float scale[OT], shift[OT], mut[IT], ist[IT];
+#pragma unroll
+  for (int ct = 0; ct < OT; ++ct)
+    {
+      scale[ct] = norm[2 * IN + 16 * ct + r];
+      shift[ct] = norm[2 * IN + OUT + 16 * ct + r];
+    }
+#pragma unroll
+  for (int rt = 0; rt < IT; ++rt)
+    {
+      mut[rt] = norm[16 * rt + r];
+      ist[rt] = norm[IN + 16 * rt + r];
+    }
+  const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+  f32x4 g1[IT][HT], g2[HT][HT], g3[HT][HT], g4[HT][OT];
+  float d1[HT], d2[HT], d3[HT], d4[OT];  // bias gradients, the lane's 4 samples of each chunk
+#pragma unroll
+  for (int ct = 0; ct < HT; ++ct)
+    {
+#pragma unroll
+      for (int rt = 0; rt < IT; ++rt)
+        g1[rt][ct] = zero;
+#pragma unroll
+      for (int rt = 0; rt < HT; ++rt)
+        {
+          g2[rt][ct] = zero;
+          g3[rt][ct] = zero;
+          if (ct < OT)
+            g4[rt][ct] = zero;
+        }
+      d1[ct] = d2[ct] = d3[ct] = 0.f;
+      if (ct < OT)
+        d4[ct] = 0.f;
+    }
   float lossacc = 0.f;
-  __syncthreads();
   const int64_t n_chunks = (n + 15) / 16;
   for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x)
     {
       const int64_t base = c * 16;
-      for (int e = l; e < 16 * IN; e += 64)
+      float t[OT][4], xt[IT][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
         {
-          const int s = e / IN, k = e % IN;
-          const int64_t row = base + s;
-          float x = 0.f;
-          if (row < n && k < n_in)
-            x = (X[row * n_in + k] - s_norm[k]) * s_norm[IN + k];
-          s_x[e] = to_bf16(x);
+          const int64_t row = base + kq + j;
+#pragma unroll
+          for (int ct = 0; ct < OT; ++ct)
+            {
+              const int o = 16 * ct + r;
+              t[ct][j] = row < n && o < n_out ? T[row * n_out + o] : shift[ct];
+            }
+#pragma unroll
+          for (int rt = 0; rt < IT; ++rt)
+            {
+              const int i = 16 * rt + r;
+              xt[rt][j] = row < n && i < n_in ? X[row * n_in + i] : mut[rt];
+            }
         }
-      for (int e = l; e < 16 * OUT; e += 64)
-        {
-          const int s = e / OUT, o = e % OUT;
-          const int64_t row = base + s;
-          s_t[e] = (row < n && o < n_out)
-                     ? (T[row * n_out + o] - s_norm[2 * IN + OUT + o]) / s_norm[2 * IN + o]
-                     : 0.f;
-        }
-      __syncthreads();
-      forward_tile(s_x, s_wt, p, s_h[0], s_h[1], s_h[2], s_z, s_y);
+      const bf16x8 x = load_inputs(X, base, n, n_in, mu, is);
+      bf16x4 h[3][HT];
+      f32x4 slope[3][HT], out[OT];
+      forward_tile(x, W, s_h, out, h, slope);
       // dL/dy of the mean squared error over the n x n_out valid outputs
-      for (int e = l; e < 16 * OUT; e += 64)
-        {
-          const int s = e / OUT, o = e % OUT;
-          const bool valid = base + s < n && o < n_out;
-          const float d = valid ? s_y[e] - s_t[e] : 0.f;
-          lossacc += d * d;
-          const float g = d * gscale;
-          s_df[0][e] = g;
-          s_d[0][e] = to_bf16(g);
-        }
-      __syncthreads();
-      // output layer: db4, dW4 = H2^T dY, dH2 = dY W4^T
-      if (l < OUT)
-        {
-          float sb = 0.f;
-          for (int s = 0; s < 16; ++s)
-            sb += s_df[0][s * OUT + l];
-          s_g[B4 + l] += sb;
-        }
+      bf16x4 dy[OT];
 #pragma unroll
-      for (int rt = 0; rt < HID / 16; ++rt)
+      for (int ct = 0; ct < OT; ++ct)
 #pragma unroll
-        for (int ct = 0; ct < OUT / 16; ++ct)
+        for (int j = 0; j < 4; ++j)
           {
-            bf16x4 a, b;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              {
-                a[j] = (short)s_h[2][(kq + j) * HID + 16 * rt + r];
-                b[j] = (short)s_d[0][(kq + j) * OUT + 16 * ct + r];
-              }
-            const f32x4 acc = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              s_g[W4 + (16 * rt + kq + j) * OUT + 16 * ct + r] += acc[j];
+            const bool valid = base + kq + j < n && 16 * ct + r < n_out;
+            const float d = valid ? out[ct][j] - (t[ct][j] - shift[ct]) / scale[ct] : 0.f;
+            lossacc += d * d;
+            const float gr = d * gscale;
+            d4[ct] += gr;
+            const bf16 b = to_bf16(gr);
+            dy[ct][j] = (short)b;
+            s_h[1][(kq + j) * LDT + 16 * ct + r] = b;
           }
+      tile_fence();
+      // output layer: dW4 = H3^T dY, dZ3 = (dY W4^T) gelu'
+      f32x4 acc[HT];
+      {
+        const bf16x8 a = load8(s_h[1] + r * LDT + k8);
 #pragma unroll
-      for (int ct = 0; ct < HID / 16; ++ct)
-        {
-          f32x4 acc{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < HT; ++ct)
+          acc[ct] = mfma32(a, v4[ct], zero);
+      }
 #pragma unroll
-          for (int kk = 0; kk < OUT / 32; ++kk)
-            acc = mfma32(load8(s_d[0] + r * OUT + 32 * kk + k8),
-                         load8(s_wb + (W4 - WB0) + (16 * ct + r) * OUT + 32 * kk + k8), acc);
+      for (int rt = 0; rt < HT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < OT; ++ct)
+          g4[rt][ct] = mfma(h[2][rt], dy[ct], g4[rt][ct]);
+      // hidden layers: dZ in operand form dz, its bias sums, and as rows in LDS
+      bf16x4 dz[HT];
+      auto scaled = [&](const f32x4(&sl)[HT], float(&db)[HT], bf16 *rows) {
+#pragma unroll
+        for (int ct = 0; ct < HT; ++ct)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             {
-              const int s = kq + j, u = 16 * ct + r;
-              const float dz = acc[j] * gelu_prime(s_z[2 * 16 * HID + s * HID + u]);
-              s_df[1][s * HID + u] = dz;
-              s_d[1][s * HID + u] = to_bf16(dz);
+              const float v = acc[ct][j] * sl[ct][j];
+              db[ct] += v;
+              const bf16 b = to_bf16(v);
+              dz[ct][j] = (short)b;
+              if (rows)
+                rows[(kq + j) * LDT + 16 * ct + r] = b;
             }
-        }
-      __syncthreads();
-      // hidden layers 3 and 2: db, dW = H_in^T dZ, dZ_in = (dZ W^T) * gelu'(Z_in)
+      };
+      scaled(slope[2], d3, s_h[0]);
+      tile_fence();
+      tile_product<HT>(s_h[0], v3, acc);
 #pragma unroll
-      for (int layer = 2; layer >= 1; --layer)
+      for (int rt = 0; rt < HT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < HT; ++ct)
+          g3[rt][ct] = mfma(h[1][rt], dz[ct], g3[rt][ct]);
+      scaled(slope[1], d2, s_h[1]);
+      tile_fence();
+      tile_product<HT>(s_h[1], v2, acc);
+#pragma unroll
+      for (int rt = 0; rt < HT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < HT; ++ct)
+          g2[rt][ct] = mfma(h[0][rt], dz[ct], g2[rt][ct]);
+      scaled(slope[0], d1, nullptr);
+      // first layer: dW1 = X^T dZ1
+#pragma unroll
+      for (int rt = 0; rt < IT; ++rt)
         {
-          const int cur = layer == 2 ? 1 : 0, nxt = 1 - cur;
-          const int Wo = layer == 2 ? W3 : W2, Bo = layer == 2 ? B3 : B2;
-          const bf16 *Hin = s_h[layer - 1];
-          {
-            float sb = 0.f;
-            for (int s = 0; s < 16; ++s)
-              sb += s_df[cur][s * HID + l];
-            s_g[Bo + l] += sb;
-          }
+          bf16x4 a;
 #pragma unroll
-          for (int rt = 0; rt < HID / 16; ++rt)
+          for (int j = 0; j < 4; ++j)
+            a[j] = (short)to_bf16((xt[rt][j] - mut[rt]) * ist[rt]);
 #pragma unroll
-            for (int ct = 0; ct < HID / 16; ++ct)
-              {
-                bf16x4 a, b;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                  {
-                    a[j] = (short)Hin[(kq + j) * HID + 16 * rt + r];
-                    b[j] = (short)s_d[cur][(kq + j) * HID + 16 * ct + r];
-                  }
-                const f32x4 acc = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                  s_g[Wo + (16 * rt + kq + j) * HID + 16 * ct + r] += acc[j];
-              }
-#pragma unroll
-          for (int ct = 0; ct < HID / 16; ++ct)
-            {
-              f32x4 acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-              for (int kk = 0; kk < HID / 32; ++kk)
-                acc = mfma32(load8(s_d[cur] + r * HID + 32 * kk + k8),
-                             load8(s_wb + (Wo - WB0) + (16 * ct + r) * HID + 32 * kk + k8),
-                             acc);
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                {
-                  const int s = kq + j, u = 16 * ct + r;
-                  const float dz =
-                    acc[j] * gelu_prime(s_z[(layer - 1) * 16 * HID + s * HID + u]);
-                  s_df[nxt][s * HID + u] = dz;
-                  s_d[nxt][s * HID + u] = to_bf16(dz);
-                }
-            }
-          __syncthreads();
+          for (int ct = 0; ct < HT; ++ct)
+            g1[rt][ct] = mfma(a, dz[ct], g1[rt][ct]);
         }
-      // first layer (dZ1 in buffer 1): db1, dW1 = X^T dZ1
+      tile_fence();
+    }
+  float *out = partial + (size_t)blockIdx.x * NPARAM;
+#pragma unroll
+  for (int ct = 0; ct < HT; ++ct)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
       {
-        float sb = 0.f;
-        for (int s = 0; s < 16; ++s)
-          sb += s_df[1][s * HID + l];
-        s_g[B1 + l] += sb;
-      }
 #pragma unroll
-      for (int rt = 0; rt < IN / 16; ++rt)
+        for (int rt = 0; rt < IT; ++rt)
+          out[W1 + (16 * rt + kq + j) * HID + 16 * ct + r] = g1[rt][ct][j];
 #pragma unroll
-        for (int ct = 0; ct < HID / 16; ++ct)
+        for (int rt = 0; rt < HT; ++rt)
           {
-            bf16x4 a, b;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              {
-                a[j] = (short)s_x[(kq + j) * IN + 16 * rt + r];
-                b[j] = (short)s_d[1][(kq + j) * HID + 16 * ct + r];
-              }
-            const f32x4 acc = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              s_g[W1 + (16 * rt + kq + j) * HID + 16 * ct + r] += acc[j];
+            out[W2 + (16 * rt + kq + j) * HID + 16 * ct + r] = g2[rt][ct][j];
+            out[W3 + (16 * rt + kq + j) * HID + 16 * ct + r] = g3[rt][ct][j];
+            if (ct < OT)
+              out[W4 + (16 * rt + kq + j) * OUT + 16 * ct + r] = g4[rt][ct][j];
           }
-      __syncthreads();
-    }
-  for (int i = l; i < NPARAM; i += 64)
-    partial[(size_t)blockIdx.x * NPARAM + i] = s_g[i];
-  s_loss[l] = lossacc;
-  __syncthreads();
-  if (l == 0)
+      }
+  auto over_samples = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+#pragma unroll
+  for (int ct = 0; ct < HT; ++ct)
     {
-      float s = 0.f;
-      for (int i = 0; i < 64; ++i)
-        s += s_loss[i];
-      lossp[blockIdx.x] = s;
+      const float s1 = over_samples(d1[ct]), s2 = over_samples(d2[ct]);
+      const float s3 = over_samples(d3[ct]), s4 = ct < OT ? over_samples(d4[ct % OT]) : 0.f;
+      if (g == 0)
+        {
+          out[B1 + 16 * ct + r] = s1;
+          out[B2 + 16 * ct + r] = s2;
+          out[B3 + 16 * ct + r] = s3;
+          if (ct < OT)
+            out[B4 + 16 * ct + r] = s4;
+        }
     }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    lossacc += __shfl_xor(lossacc, off);
+  if (l == 0)
+    lossp[blockIdx.x] = lossacc;
 }
 
-__global__ void k_mlp_reduce(const float *__restrict__ partial, int G, float *__restrict__ grad)
+// grad = sum of the G partials.  A workgroup takes 32 parameters: 8 threads share one parameter's
+// partials (every eighth each, 8 loads in flight) and their sums are added in order, so the
+// result does not depend on the launch.  G = 256: 54 us with one thread and one load at a time per
+// parameter, 5.2 us.
+constexpr int RED_PARAMS = 32, RED_LANES = 8;
+__global__ __launch_bounds__(RED_PARAMS *RED_LANES) void k_mlp_reduce(
+  const float *__restrict__ partial, int G, float *__restrict__ grad)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= NPARAM)
-    return;
+  __shared__ float part[RED_LANES][RED_PARAMS];
+  const int q = threadIdx.x % RED_PARAMS, y = threadIdx.x / RED_PARAMS;
+  const int i = blockIdx.x * RED_PARAMS + q;
   float s = 0.f;
-  for (int b = 0; b < G; ++b)
-    s += partial[(size_t)b * NPARAM + i];
-  grad[i] = s;
+  if (i < NPARAM)
+    {
+      int b = y;
+      for (; b + 7 * RED_LANES < G; b += 8 * RED_LANES)
+        {
+          float v[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            v[k] = partial[(size_t)(b + k * RED_LANES) * NPARAM + i];
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            s += v[k];
+        }
+      for (; b < G; b += RED_LANES)
+        s += partial[(size_t)b * NPARAM + i];
+    }
+  part[y][q] = s;
+  __syncthreads();
+  if (y == 0 && i < NPARAM)
+    {
+#pragma unroll
+      for (int k = 1; k < RED_LANES; ++k)
+        s += part[k][q];
+      grad[i] = s;
+    }
 }
 
 __device__ inline int transposed_index(int i)
@@ -293,43 +365,41 @@ __global__ void k_mlp_adam(float *__restrict__ p, float *__restrict__ m, float *
     wt[t] = to_bf16(w);
 }
 
-__global__ __launch_bounds__(256) void k_mlp_forward(const float *__restrict__ p,
-                                                     const bf16 *__restrict__ wt_g,
-                                                     const float *__restrict__ norm,
-                                                     int64_t n, int n_in, int n_out,
-                                                     const float *__restrict__ X,
-                                                     float *__restrict__ Y)
+// rows of tiles blockIdx.x, blockIdx.x + gridDim.x, ... of 16; one wave, weights in registers
+__global__ __launch_bounds__(64) void k_mlp_forward(const float *__restrict__ p,
+                                                    const bf16 *__restrict__ wt,
+                                                    const float *__restrict__ norm, int64_t n,
+                                                    int n_in, int n_out,
+                                                    const float *__restrict__ X,
+                                                    float *__restrict__ Y)
 {
-  __shared__ __attribute__((aligned(16))) bf16 s_wt[NT];
-  __shared__ __attribute__((aligned(16))) bf16 s_x[4][16 * IN];
-  __shared__ __attribute__((aligned(16))) bf16 s_h[4][3][16 * HID];
-  __shared__ float s_y[4][16 * OUT];
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  for (int i = threadIdx.x; i < NT; i += 256)
-    s_wt[i] = wt_g[i];
-  __syncthreads();
-  for (int tile = 0; tile < 4; ++tile)
+  __shared__ __attribute__((aligned(16))) bf16 s_h[2][16 * LDT];
+  const int l = threadIdx.x, r = l & 15, kq = (l >> 4) * 4, k8 = (l >> 4) * 8;
+  ForwardWeights W;
+  W.load(wt, p);
+  float mu[8], is[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
     {
-      const int64_t base = (int64_t)blockIdx.x * 256 + (int64_t)(w * 4 + tile) * 16;
-      for (int e = l; e < 16 * IN; e += 64)
-        {
-          const int s = e / IN, k = e % IN;
-          const int64_t row = base + s;
-          float x = 0.f;
-          if (row < n && k < n_in)
-            x = (X[row * n_in + k] - norm[k]) * norm[IN + k];
-          s_x[w][e] = to_bf16(x);
-        }
-      __syncthreads();
-      forward_tile(s_x[w], s_wt, p, s_h[w][0], s_h[w][1], s_h[w][2], nullptr, s_y[w]);
-      for (int e = l; e < 16 * OUT; e += 64)
-        {
-          const int s = e / OUT, o = e % OUT;
-          const int64_t row = base + s;
-          if (row < n && o < n_out)
-            Y[row * n_out + o] = output_value(s_y[w][e], norm, o);
-        }
-      __syncthreads();
+      mu[j] = norm[k8 + j];
+      is[j] = norm[IN + k8 + j];
+    }
+  for (int64_t tile = blockIdx.x; tile * 16 < n; tile += gridDim.x)
+    {
+      const bf16x8 x = load_inputs(X, tile * 16, n, n_in, mu, is);
+      f32x4 out[OUT / 16];
+      forward_tile(x, W, s_h, out);
+#pragma unroll
+      for (int ct = 0; ct < OUT / 16; ++ct)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          {
+            const int64_t row = tile * 16 + kq + j;
+            const int o = 16 * ct + r;
+            if (row < n && o < n_out)
+              Y[row * n_out + o] = output_value(out[ct][j], norm, o);
+          }
+      tile_fence();
     }
 }
 
@@ -389,8 +459,8 @@ int grad_launch(oc_mlp *m, int64_t n, const float *x, const float *t, hipStream_
   const float gscale = 2.0f / (float)((double)n * (double)m->n_out);
   hipLaunchKernelGGL(k_mlp_grad, dim3(*G), dim3(64), 0, s, m->p, m->wt, m->wb, m->norm, n,
                      m->n_in, m->n_out, x, t, gscale, m->partial, m->lossp);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + 255) / 256), dim3(256), 0, s, m->partial, *G,
-                     m->grad);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + RED_PARAMS - 1) / RED_PARAMS),
+                     dim3(RED_PARAMS * RED_LANES), 0, s, m->partial, *G, m->grad);
   MLP_TRY(hipGetLastError());
   return OC_OK;
 }
@@ -563,7 +633,8 @@ int oc_mlp_forward(oc_mlp *m, int64_t n, const float *x, float *y, void *stream)
     }
   if (n == 0)
     return OC_OK;
-  hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+  const int64_t tiles = (n + 15) / 16;
+  hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)std::min<int64_t>(tiles, 4096)), dim3(64), 0,
                      (hipStream_t)stream, m->p, m->wt, m->norm, n, m->n_in, m->n_out, x, y);
   MLP_TRY(hipGetLastError());
   return OC_OK;

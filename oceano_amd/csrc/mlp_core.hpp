@@ -66,15 +66,6 @@ __host__ __device__ inline float from_bf16(bf16 h)
   return f;
 }
 
-// GELU, erf form, and its derivative
-__device__ inline float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-
-__device__ inline float gelu_prime(float x)
-{
-  return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) +
-         x * 0.39894228040143268f * expf(-0.5f * x * x);
-}
-
 __device__ inline f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c)
 {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -88,75 +79,126 @@ __device__ inline f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 // the 8 consecutive BF16 values at p (16-byte aligned) as an MFMA operand
 __device__ inline bf16x8 load8(const bf16 *p) { return *(const bf16x8 *)p; }
 
-// acc[ct] = A[16 x K] * W for the N / 16 column tiles (K a multiple of 32); A row-major with
-// leading dimension K in LDS, W given transposed (WT[n][k], leading dimension K).  The k
-// order is fixed, so a row's result does not depend on the other rows of the tile.
-template <int K, int N>
-__device__ inline void dense_tile(const bf16 *A, const bf16 *WT, f32x4 (&acc)[N / 16])
+// A wave works on tiles of 16 samples with every weight in registers: the B operand of a
+// column tile and 32-deep step is 16 consecutive bytes of the transposed weights per lane, so
+// one lane holds the whole network in 24 loads of 16 bytes (96 registers), issued at once.  The
+// alternative, a copy in LDS, costs each workgroup 24 KiB of staging before its first product:
+// the in-stage inference on 2,500 cells took 33.0 us with it, 9.6 us this way.
+struct ForwardWeights
 {
-  static_assert(K % 32 == 0, "contraction depth must be a multiple of 32");
+  bf16x8 w1[HID / 16], w2[HID / 16 * 2], w3[HID / 16 * 2], w4[OUT / 16 * 2];
+  float b1[HID / 16], b2[HID / 16], b3[HID / 16], b4[OUT / 16];
+
+  // wt: transposed BF16 weights, p: FP32 parameters (biases), both in global memory
+  __device__ __forceinline__ void load(const bf16 *__restrict__ wt, const float *__restrict__ p)
+  {
+    const int l = threadIdx.x & 63, r = l & 15, k8 = (l >> 4) * 8;
+#pragma unroll
+    for (int ct = 0; ct < HID / 16; ++ct)
+      {
+        w1[ct] = load8(wt + T1 + (16 * ct + r) * IN + k8);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+          {
+            w2[2 * ct + kk] = load8(wt + T2 + (16 * ct + r) * HID + 32 * kk + k8);
+            w3[2 * ct + kk] = load8(wt + T3 + (16 * ct + r) * HID + 32 * kk + k8);
+          }
+        b1[ct] = p[B1 + 16 * ct + r];
+        b2[ct] = p[B2 + 16 * ct + r];
+        b3[ct] = p[B3 + 16 * ct + r];
+      }
+#pragma unroll
+    for (int ct = 0; ct < OUT / 16; ++ct)
+      {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+          w4[2 * ct + kk] = load8(wt + T4 + (16 * ct + r) * HID + 32 * kk + k8);
+        b4[ct] = p[B4 + 16 * ct + r];
+      }
+  }
+};
+
+// row stride of a 16 x 64 activation tile in LDS: 16 bytes of padding spread the 16 rows that an
+// operand read touches over the banks
+constexpr int LDT = HID + 8;
+
+// orders this wave's LDS writes before its reads by other lanes (the wave owns the tile)
+__device__ __forceinline__ void tile_fence()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc[ct] = A[16 x 64] W for NC column tiles, A in LDS (row stride LDT); the k order is fixed, so
+// a row's result does not depend on the other rows of the tile
+template <int NC>
+__device__ __forceinline__ void tile_product(const bf16 *A, const bf16x8 (&w)[2 * NC],
+                                             f32x4 (&acc)[NC])
+{
   const int l = threadIdx.x & 63, r = l & 15, k8 = (l >> 4) * 8;
 #pragma unroll
-  for (int ct = 0; ct < N / 16; ++ct)
+  for (int ct = 0; ct < NC; ++ct)
     acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int kk = 0; kk < K / 32; ++kk)
+  for (int kk = 0; kk < 2; ++kk)
     {
-      const bf16x8 a = load8(A + r * K + 32 * kk + k8);
+      const bf16x8 a = load8(A + r * LDT + 32 * kk + k8);
 #pragma unroll
-      for (int ct = 0; ct < N / 16; ++ct)
-        {
-          const bf16x8 b = load8(WT + (16 * ct + r) * K + 32 * kk + k8);
-          acc[ct] = mfma32(a, b, acc[ct]);
-        }
+      for (int ct = 0; ct < NC; ++ct)
+        acc[ct] = mfma32(a, w[2 * ct + kk], acc[ct]);
     }
 }
 
-// hidden layer epilogue: z = acc + bias, H = bf16(gelu(z)) (and z kept when Z != nullptr)
-template <int N>
-__device__ inline void hidden_epilogue(const f32x4 (&acc)[N / 16], const float *bias, bf16 *H,
-                                       float *Z)
+// bias and GELU of a layer: the BF16 activations h of the lane's accumulator entries, also into
+// the LDS tile H; slope: the GELU derivatives there (null: not needed)
+__device__ __forceinline__ void hidden_layer(const f32x4 (&acc)[HID / 16],
+                                             const float (&bias)[HID / 16], bf16 *H,
+                                             bf16x4 (*h)[HID / 16], f32x4 (*slope)[HID / 16])
 {
   const int l = threadIdx.x & 63, r = l & 15, kq = (l >> 4) * 4;
 #pragma unroll
-  for (int ct = 0; ct < N / 16; ++ct)
+  for (int ct = 0; ct < HID / 16; ++ct)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       {
-        const int row = kq + j, col = 16 * ct + r;
-        const float z = acc[ct][j] + bias[col];
-        if (Z)
-          Z[row * N + col] = z;
-        H[row * N + col] = to_bf16(gelu(z));
+        const float z = acc[ct][j] + bias[ct];
+        const float e = erff(z * 0.70710678118654752f);
+        const bf16 v = to_bf16(0.5f * z * (1.0f + e));
+        H[(kq + j) * LDT + 16 * ct + r] = v;
+        if (h)
+          (*h)[ct][j] = (short)v;
+        if (slope)
+          (*slope)[ct][j] = 0.5f * (1.0f + e) + z * 0.39894228040143268f * expf(-0.5f * z * z);
       }
 }
 
-// forward of one 16-row tile whose normalised BF16 inputs are in X (16 x IN): Y (16 x OUT)
-// gets the network output (before de-normalisation); H0..H2 (16 x HID) the BF16 hidden
-// activations, Z (3 x 16 x HID, may be null) the pre-activations.  wt: transposed BF16
-// weights (LDS), p: FP32 parameters (for the biases).
-__device__ inline void forward_tile(const bf16 *X, const bf16 *wt, const float *p, bf16 *H0,
-                                    bf16 *H1, bf16 *H2, float *Z, float *Y)
+// forward of one tile: x the A operand of its normalised BF16 inputs (row l % 16, inputs
+// 8 (l / 16) ..), H two LDS tiles of the wave; out: entries (row 4 (l / 16) + j, output 16 ct +
+// l % 16) before de-normalisation.  h, slope (may be null): per hidden layer, see hidden_layer
+__device__ __forceinline__ void forward_tile(bf16x8 x, const ForwardWeights &W, bf16 (*H)[16 * LDT],
+                                             f32x4 (&out)[OUT / 16],
+                                             bf16x4 (*h)[HID / 16] = nullptr,
+                                             f32x4 (*slope)[HID / 16] = nullptr)
 {
   f32x4 acc[HID / 16];
-  dense_tile<IN, HID>(X, wt + T1, acc);
-  hidden_epilogue<HID>(acc, p + B1, H0, Z);
-  __syncthreads();
-  dense_tile<HID, HID>(H0, wt + T2, acc);
-  hidden_epilogue<HID>(acc, p + B2, H1, Z ? Z + 16 * HID : nullptr);
-  __syncthreads();
-  dense_tile<HID, HID>(H1, wt + T3, acc);
-  hidden_epilogue<HID>(acc, p + B3, H2, Z ? Z + 32 * HID : nullptr);
-  __syncthreads();
-  f32x4 out[OUT / 16];
-  dense_tile<HID, OUT>(H2, wt + T4, out);
-  const int l = threadIdx.x & 63, r = l & 15, kq = (l >> 4) * 4;
+#pragma unroll
+  for (int ct = 0; ct < HID / 16; ++ct)
+    acc[ct] = mfma32(x, W.w1[ct], f32x4{0.f, 0.f, 0.f, 0.f});
+  hidden_layer(acc, W.b1, H[0], h, slope);
+  tile_fence();
+  tile_product<HID / 16>(H[0], W.w2, acc);
+  hidden_layer(acc, W.b2, H[1], h ? h + 1 : nullptr, slope ? slope + 1 : nullptr);
+  tile_fence();
+  tile_product<HID / 16>(H[1], W.w3, acc);
+  hidden_layer(acc, W.b3, H[0], h ? h + 2 : nullptr, slope ? slope + 2 : nullptr);
+  tile_fence();
+  tile_product<OUT / 16>(H[0], W.w4, out);
 #pragma unroll
   for (int ct = 0; ct < OUT / 16; ++ct)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      Y[(kq + j) * OUT + 16 * ct + r] = out[ct][j] + p[B4 + 16 * ct + r];
-  __syncthreads();
+      out[ct][j] += W.b4[ct];
 }
 
 }  // namespace mlp
