@@ -24,15 +24,22 @@ namespace oceano {
 
 namespace {
 
-// The arguments of all groups are written to device memory by a one-thread kernel ahead of
+// The arguments of all groups are written to device memory by a small kernel ahead of
 // the stage kernel (in stream order, so a captured graph replays both): the stage kernel
 // reads the group it runs through a pointer, with uniform (scalar) loads.  Indexing the
 // by-value argument block by a run-time group index instead makes the compiler copy the
-// whole block to per-lane scratch memory.
-__global__ void k_put_multi_args(MultiArgs A, MultiArgs *dst)
+// whole block to per-lane scratch memory.  The words are copied by the workgroup's threads from
+// the kernel's argument segment, where A comes first: 4.6 us, against 7.2 us for one thread
+// copying A, ahead of a stage of 51 us.
+__global__ __launch_bounds__(256) void k_put_multi_args(MultiArgs A, MultiArgs *dst)
 {
-  if (threadIdx.x == 0)
-    *dst = A;
+  static_assert(sizeof(MultiArgs) % sizeof(int) == 0, "copied as words");
+  typedef __attribute__((address_space(4))) const int cint;
+  const cint *src = (const cint *)__builtin_amdgcn_kernarg_segment_ptr();
+  int *to = reinterpret_cast<int *>(dst);
+#pragma unroll
+  for (int i = threadIdx.x; i < (int)(sizeof(MultiArgs) / sizeof(int)); i += 256)
+    to[i] = src[i];
 }
 
 template <int P, typename R>
@@ -173,7 +180,7 @@ int stage_multi(int n, oc_dg *const *ops, const OpArgs *O, uint32_t stage,
   A.start[n] = start;
   const bool mixed = ops[0]->precision == OC_PRECISION_MIXED;
   MultiArgs *dA = ops[0]->d_multi_args;
-  hipLaunchKernelGGL(k_put_multi_args, dim3(1), dim3(CB), 0, s, A, dA);
+  hipLaunchKernelGGL(k_put_multi_args, dim3(1), dim3(256), 0, s, A, dA);
   HIP_TRY(hipGetLastError());
   if (paired && mixed)
     hipLaunchKernelGGL(k_stage_multi_pair<float>, dim3(start), dim3(2 * CB), 0, s, dA);
