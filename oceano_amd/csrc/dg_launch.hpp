@@ -99,7 +99,12 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
       timed_begin(op, s, &ev);
       const int items = 2 * op->NB;
       if (visc)
-        hipLaunchKernelGGL((k_stage<P, true, R, 1>), dim3(items), block, 0, s, O, H, Q);
+        {
+          if constexpr (std::is_same<R, double>::value)
+            hipLaunchKernelGGL((k_stage_pair<P, R, false, true>), grid, dim3(2 * CB), 0, s, O, H, Q);
+          else
+            hipLaunchKernelGGL((k_stage<P, true, R, 1>), dim3(items), block, 0, s, O, H, Q);
+        }
       else if (op->paired_items)
         {
           if (std::is_same<R, float>::value && P <= 3)
@@ -176,26 +181,39 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
                      hipStream_t s)
 {
   const dim3 grid(op->NB), block(CB);
-  if (invert)
-    hipLaunchKernelGGL((k_height_rhs<P, true, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
-  else
-    hipLaunchKernelGGL((k_height_rhs<P, false, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
+  const bool visc = O.nu != 0.0;
   StageArgs S{};
   S.src_h = src_h;
   S.src_q = src_q;
   S.src_v = src_v;
   S.dst = dst_q;
-  const bool visc = O.nu != 0.0;
-  if (invert)
+  if constexpr (std::is_same<R, double>::value)
     {
-      if (visc)
-        hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
+      // one launch of paired items.  The FP32 integrals keep two launches: their results carry
+      // the order of summation of the unpaired items
+      StageArgs H = S;
+      H.dst = dst_h;
+      const dim3 pair(2 * CB);
+      if (invert && visc)
+        hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 1>), grid, pair, 0, s, O, H, S);
+      else if (invert)
+        hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 1>), grid, pair, 0, s, O, H, S);
+      else if (visc)
+        hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 2>), grid, pair, 0, s, O, H, S);
       else
-        hipLaunchKernelGGL((k_discharge<P, false, 1, R>), grid, block, 0, s, O, S);
+        hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 2>), grid, pair, 0, s, O, H, S);
     }
   else
     {
-      if (visc)
+      if (invert)
+        hipLaunchKernelGGL((k_height_rhs<P, true, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
+      else
+        hipLaunchKernelGGL((k_height_rhs<P, false, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
+      if (invert && visc)
+        hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
+      else if (invert)
+        hipLaunchKernelGGL((k_discharge<P, false, 1, R>), grid, block, 0, s, O, S);
+      else if (visc)
         hipLaunchKernelGGL((k_discharge<P, true, 2, R>), grid, block, 0, s, O, S);
       else
         hipLaunchKernelGGL((k_discharge<P, false, 2, R>), grid, block, 0, s, O, S);

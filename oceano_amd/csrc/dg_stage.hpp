@@ -1213,9 +1213,7 @@ __device__ __forceinline__ void discharge_block(const OpArgs &O, const StageArgs
       // faces 2 and 3 for both equations (pair_exchange); the LDS copy of the batch's own
       // data staged above is the height wave's too (read after this barrier, until the
       // exchange)
-      static_assert(!VISC && (MODE == 0 || MODE == 4),
-                    "paired items: inviscid stage (explicit, or the additive stage's explicit "
-                    "momentum integrals)");
+      static_assert(MODE != 3, "paired items: no split path");
       __syncthreads();
       R A[3][ND];
 #pragma unroll
@@ -2050,7 +2048,8 @@ __global__ __launch_bounds__(CB) void k_depth_deferred(OpArgs O, StageArgs S)
 // L_zeta, front and depth solve of one batch of cells in one pass: L_zeta stays in
 // registers for the front (it is also written out as ki_h[stage+1] for later stages).
 // IN32 / S.out32 as for discharge_block (the zeta register's centres included)
-template <int P, typename R, bool PAIR = false, bool IN32 = false>
+// MODE 1, 2 (paired only): apply and rhs, M^-1 L_zeta or L_zeta into the FP64 vector S.dst
+template <int P, typename R, bool PAIR = false, bool IN32 = false, int MODE = 0>
 __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageArgs &S,
                                                    int batch, float *lds, R *xch = nullptr,
                                                    const R *own = nullptr)
@@ -2140,7 +2139,7 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
       // cells at p = 2, FP64 83 -> 79 us.  At p = 1 both waves arrive together and it would
       // only delay the other (819,200 cells, mixed: 300 -> 302 us)
       pair_exchange<P, R, 0>(A, xch, [&] {
-        if constexpr (P >= 2)
+        if constexpr (P >= 2 && MODE == 0)
           {
             prepare_front();
             prepare_depth();
@@ -2160,6 +2159,18 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
       height_operator<P, R>(O, basis<R>(P), physics<R>(O), batch, lane, R(hx), R(hy),
                             (const R *)Zo, (const R *)QX, (const R *)QY, zc, S.src_h,
                             S.src_q, Racc);
+    }
+  if constexpr (MODE != 0)
+    {
+      if (active)
+        {
+          if (MODE == 1)
+            tensor_inverse<P>(basis<R>(P), Racc[0], R(1) / R(area));
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            S.dst[vix(batch, 1, 0, ND, i, lane)] = double(Racc[0][i]);
+        }
+      return;
     }
   constexpr bool PREPARED = PAIR && P >= 2;
   if (active)
@@ -2293,10 +2304,10 @@ __host__ __device__ constexpr int pair_height_words()
   return (pair_xch_offset<P, R>() + pair_xch_words<P>() + 63) / 64 * 64;
 }
 
-template <int P, typename R>
+template <int P, typename R, bool VISC = false>
 __host__ __device__ constexpr int pair_lds_words()
 {
-  return pair_height_words<P, R>() + discharge_lds_words<P, false>();
+  return pair_height_words<P, R>() + discharge_lds_words<P, VISC>();
 }
 
 // Which wave of a paired workgroup runs the height item: wave item_kind(blockIdx.x), the
@@ -2318,19 +2329,20 @@ __device__ __forceinline__ bool pair_height_wave()
 // IN32: the stage input comes in its centred FP32 form (c32_values, c32_centres; the device
 // time loop's intermediate stages); a compile-time variant, so that neither form's kernel
 // carries the other's loads
-template <int P, typename R, bool IN32 = false>
+// MODE 1, 2: apply (M^-1 L) and rhs (L) of Q.src_h, Q.src_q into H.dst, Q.dst
+template <int P, typename R, bool IN32 = false, bool VISC = false, int MODE = 0>
 __global__ __launch_bounds__(2 * CB, (stage_min_waves<P, false, R>())) void k_stage_pair(
   OpArgs O, StageArgs H, StageArgs Q)
 {
-  __shared__ __align__(16) R lds[pair_lds_words<P, R>()];
+  __shared__ __align__(16) R lds[pair_lds_words<P, R, VISC>()];
   const int batch = logical_batch(blockIdx.x, O.n_batches, O.xcd_swizzle);
   R *xch = lds + pair_xch_offset<P, R>();
   R *dlds = lds + pair_height_words<P, R>();
   if (pair_height_wave())
-    height_stage_block<P, R, true, IN32>(O, H, batch, reinterpret_cast<float *>(lds), xch,
-                                         dlds);
+    height_stage_block<P, R, true, IN32, MODE>(O, H, batch, reinterpret_cast<float *>(lds), xch,
+                                               dlds);
   else
-    discharge_block<P, false, 0, R, true, IN32>(O, Q, batch, dlds, xch);
+    discharge_block<P, VISC, MODE, R, true, IN32>(O, Q, batch, dlds, xch);
 }
 
 }  // namespace oceano
