@@ -100,7 +100,11 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
       const int items = 2 * op->NB;
       if (visc)
         {
-          if constexpr (std::is_same<R, double>::value)
+          // paired in FP64 at p <= 2 (RK4 step of 12,800 cells at p = 1 43 -> 35 us, of 51,200 at
+          // p = 2 138 -> 129 us); at p >= 3 the cell term's gradients of the velocity fill two
+          // waves' registers and the unpaired items at one wave per SIMD are faster (26,000 hanging
+          // cells at p = 3: 196 us a step, paired 225; 5,000 at p = 4: 264, paired 279)
+          if constexpr (std::is_same<R, double>::value && P <= 2)
             hipLaunchKernelGGL((k_stage_pair<P, R, false, true>), grid, dim3(2 * CB), 0, s, O, H, Q);
           else
             hipLaunchKernelGGL((k_stage<P, true, R, 1>), dim3(items), block, 0, s, O, H, Q);
