@@ -44,7 +44,7 @@ __device__ __forceinline__ void stiff_source(const OpArgs &O, const Basis<R> &T,
                                              R (&Ry)[(P + 1) * (P + 1)])
 {
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P);
-  const Phys<R> M = physics<R>(O);
+  const auto M = physics<R>(O);
 #pragma unroll
   for (int k = 0; k < ND; ++k)
     Rx[k] = Ry[k] = 0;
@@ -220,7 +220,7 @@ __device__ __forceinline__ void ark_update_cell(const OpArgs &O, const ArkArgs &
       iw[a + N1 * b] = 1. / (T.wn[a] * T.wn[b] * area);
   if (!A.last)
     {
-      const Phys<double> M = physics<double>(O);
+      const auto M = physics<double>(O);
       double U[ND], z[ND], qx[ND], qy[ND];
 #pragma unroll
       for (int k = 0; k < ND; ++k)

@@ -100,7 +100,42 @@ struct OpArgs
   unsigned long long *defer;  // mixed path: per batch, lanes whose depth solve is deferred
   unsigned int *sweeps;       // per batch: Jacobi sweeps of the last stage (sum over lanes)
   const double *closure;  // [batch][2][nd][lane] M^-1-form momentum source, or nullptr
+  // terms known when a kernel is compiled (PlainArgs, ManningArgs); here none are
+  static constexpr bool FLAT = false;
+  __host__ __device__ bool friction() const { return has_friction != 0; }
+  __host__ __device__ bool wind() const { return has_wind != 0; }
+  __host__ __device__ bool coriolis() const { return has_coriolis != 0; }
 };
+
+// The same arguments where the problem's data settle which terms there are.  Tested at run
+// time, every term ends a basic block at every quadrature point: the points of a row (or of a face)
+// then cannot be interleaved, and with one to three waves per SIMD each point waits out its own
+// chain of dependent instructions.  RK4 step of 97,280 cells at p = 3 mixed 177 -> 159 us, FP64
+// 355 -> 320 us; of 12,800 at p = 1 FP64 40 -> 35 us; channel of 2,500 at p = 2 FP64 79 -> 70 us.
+//   PlainArgs    no friction, wind or Coriolis force, every bed field uniform
+//   ManningArgs  friction, neither wind nor Coriolis force, any bed
+struct PlainArgs : OpArgs
+{
+  static constexpr bool FLAT = true;
+  __host__ __device__ static constexpr bool friction() { return false; }
+  __host__ __device__ static constexpr bool wind() { return false; }
+  __host__ __device__ static constexpr bool coriolis() { return false; }
+};
+struct ManningArgs : OpArgs
+{
+  __host__ __device__ static constexpr bool friction() { return true; }
+  __host__ __device__ static constexpr bool wind() { return false; }
+  __host__ __device__ static constexpr bool coriolis() { return false; }
+};
+inline bool is_plain(const OpArgs &O)
+{
+  return !O.has_friction && !O.has_wind && !O.has_coriolis && !O.cell0[0].ptr && !O.cell1.ptr &&
+         !O.facez.ptr && !O.bdryz.ptr;
+}
+inline bool is_manning(const OpArgs &O)
+{
+  return O.has_friction && !O.has_wind && !O.has_coriolis;
+}
 
 struct StageArgs
 {
@@ -203,26 +238,74 @@ __device__ __forceinline__ double fld(const Field &f, size_t i)
 // the compiler then parks the argument block in VGPR lanes and restores a whole group of
 // 16 SGPRs (one v_readlane each) at every read of a field inside a loop.  Copied into
 // VGPRs once, a read is a select (or the load) and nothing more.
-template <typename R>
+// FLAT: known to be uniform.
+template <typename R, bool FLAT = false>
 struct FieldV
 {
   const double *ptr;
   R cval;
   bool stored;
 };
-
 template <typename R>
-__device__ __forceinline__ FieldV<R> in_vgprs(const Field &f)
+struct FieldV<R, true>
 {
-  FieldV<R> v{f.ptr, R(f.cval), f.ptr != nullptr};
-  asm volatile("" : "+v"(v.ptr), "+v"(v.cval));
-  return v;
+  R cval;
+};
+
+template <typename R, typename OA>
+__device__ __forceinline__ FieldV<R, OA::FLAT> in_vgprs(const OA &, const Field &f)
+{
+  if constexpr (OA::FLAT)
+    return {R(f.cval)};
+  else
+    {
+      FieldV<R> v{f.ptr, R(f.cval), f.ptr != nullptr};
+      asm volatile("" : "+v"(v.ptr), "+v"(v.cval));
+      return v;
+    }
 }
 
 template <typename R>
 __device__ __forceinline__ R fld(const FieldV<R> &f, size_t i)
 {
   return f.stored ? R(f.ptr[i]) : f.cval;
+}
+template <typename R>
+__device__ __forceinline__ R fld(const FieldV<R, true> &f, size_t)
+{
+  return f.cval;
+}
+
+// N consecutive values of a field (index i + j STRIDE), their loads in one group: read one by
+// one at their points, each would be a wait of its own
+template <int N, int STRIDE, typename R>
+__device__ __forceinline__ void fld_row(const FieldV<R> &f, size_t i, R (&v)[N])
+{
+  if (f.stored)
+    {
+      double t[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        t[j] = f.ptr[i + (size_t)j * STRIDE];
+      issue_barrier();
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        v[j] = R(t[j]);
+    }
+  else
+    {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        v[j] = f.cval;
+    }
+}
+
+template <int N, int STRIDE, typename R>
+__device__ __forceinline__ void fld_row(const FieldV<R, true> &f, size_t, R (&v)[N])
+{
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    v[j] = f.cval;
 }
 
 }  // namespace oceano

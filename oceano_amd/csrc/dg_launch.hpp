@@ -111,13 +111,24 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
         }
       else if (op->paired_items)
         {
-          if (std::is_same<R, float>::value && P <= 3)
+          constexpr bool C32 = std::is_same<R, float>::value && P <= 3;
+          if (C32)
             H.out32 = Q.out32 = op->rk_out32 && !last;
-          if (std::is_same<R, float>::value && P <= 3 && op->rk_in32)
-            hipLaunchKernelGGL((k_stage_pair<P, R, std::is_same<R, float>::value && P <= 3>),
-                               grid, dim3(2 * CB), 0, s, O, H, Q);
+          auto launch = [&](auto args) {
+            using OA = decltype(args);
+            if (C32 && op->rk_in32)
+              hipLaunchKernelGGL((k_stage_pair<P, R, C32, false, 0, OA>), grid, dim3(2 * CB), 0, s,
+                                 args, H, Q);
+            else
+              hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 0, OA>), grid, dim3(2 * CB), 0,
+                                 s, args, H, Q);
+          };
+          if (is_plain(O))
+            launch(PlainArgs{O});
+          else if (is_manning(O))
+            launch(ManningArgs{O});
           else
-            hipLaunchKernelGGL((k_stage_pair<P, R>), grid, dim3(2 * CB), 0, s, O, H, Q);
+            launch(O);
         }
       else if (op->waves_per_block == 4)
         hipLaunchKernelGGL((k_stage<P, false, R, 4>), dim3((items + 3) / 4), dim3(4 * CB), 0,

@@ -40,6 +40,25 @@ __device__ __forceinline__ double rsqrt_nr(double x)
 // FP32 (mixed path): the hardware reciprocal square root (within 1 ulp), unrefined
 __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// a b + c d.  FP32: the first product rounded, the second fused.  Which of two products a compiler
+// fuses depends on the code around them; written out, the FP32 results of the integrals do not
+// change with it
+__device__ __forceinline__ double two_products(double a, double b, double c, double d)
+{
+  return a * b + c * d;
+}
+__device__ __forceinline__ float two_products(float a, float b, float c, float d)
+{
+  return __builtin_fmaf(c, d, a * b);
+}
+
+// s + a b, the product fused
+__device__ __forceinline__ double plus_product(double s, double a, double b) { return s + a * b; }
+__device__ __forceinline__ float plus_product(float s, float a, float b)
+{
+  return __builtin_fmaf(a, b, s);
+}
+
 // sqrt(x), x >= 0, through rsqrt_nr
 __device__ __forceinline__ double sqrt_nr(double x) { return x > 0.0 ? x * rsqrt_nr(x) : x; }
 
@@ -80,7 +99,7 @@ __device__ __forceinline__ float manning_coefficient(float g, float n, float h, 
                                                      float vy)
 {
   const float inv_d = 1.f / (exp(log(h) * 0.33333333333f));
-  return g * n * n * inv_d * sqrt(vx * vx + vy * vy);
+  return g * n * n * inv_d * sqrt(two_products(vy, vy, vx, vx));
 }
 
 // a . n for the axis-aligned normals of the kernels: with one component of n zero the
@@ -96,7 +115,8 @@ __host__ __device__ __forceinline__ T dot_n(Vec2<T> a, Vec2<T> n)
   return a.x * n.x + a.y * n.y;
 }
 
-template <typename T>
+// FLAT: the bed is known to be uniform (zb_m == zb_p everywhere)
+template <typename T, bool FLAT = false>
 struct Phys
 {
   T g;
@@ -148,7 +168,9 @@ struct Phys
            T(0.5) * lambda * (zcm - zcp);
   }
 
-  // LaxFriedrichsModified::numerical_advflux_weak
+  // LaxFriedrichsModified::numerical_advflux_weak.  BOUNDARY only turns the FP32 rounding of
+  // its sums round (two_products): the boundary faces have always been summed so
+  template <bool BOUNDARY = false>
   __device__ __forceinline__ Vec2<T> adv_flux(T z_m, T z_p, Vec2<T> q_m, Vec2<T> q_p,
                                              Vec2<T> n, T zb_m, T zb_p) const
   {
@@ -165,7 +187,7 @@ struct Phys
     // advective_flux(z, hu, zb*): F[e][d] = hu_e * velocity(z, hu, zb*)_d; with a
     // continuous bathymetry zb* = zb_m = zb_p and the inverse depths are the ones above
     T sm = s_m, sp = s_p;
-    if (zb_m != zb_p)
+    if (!FLAT && zb_m != zb_p)
       {
         sm = inv_depth(hm);
         sp = inv_depth(hp);
@@ -175,8 +197,11 @@ struct Phys
     const T wn_m = dot_n(w_m, n);
     const T wn_p = dot_n(w_p, n);
     const T hl = T(0.5) * lambda;
-    return {T(0.5) * (hu_m.x * wn_m + hu_p.x * wn_p) + hl * (hu_m.x - hu_p.x),
-            T(0.5) * (hu_m.y * wn_m + hu_p.y * wn_p) + hl * (hu_m.y - hu_p.y)};
+    if (BOUNDARY)
+      return {two_products(hl, hu_m.x - hu_p.x, T(0.5), two_products(hu_p.x, wn_p, hu_m.x, wn_m)),
+              two_products(hl, hu_m.y - hu_p.y, T(0.5), two_products(hu_p.y, wn_p, hu_m.y, wn_m))};
+    return {two_products(T(0.5), two_products(hu_m.x, wn_m, hu_p.x, wn_p), hl, hu_m.x - hu_p.x),
+            two_products(T(0.5), two_products(hu_m.y, wn_m, hu_p.y, wn_p), hl, hu_m.y - hu_p.y)};
   }
 
   // NumericalFluxBase::numerical_presflux_strong, CENTER variant

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(CB) void k_velocity(OpArgs O, const double *__restr
   const int batch = blockIdx.x, lane = threadIdx.x;
   if (batch * CB + lane >= O.n_cells)
     return;
-  const Phys<double> M = physics<double>(O);
+  const auto M = physics<double>(O);
   double U[ND], z[ND], qx[ND], qy[ND];
   // Sn is [n1][n1]; widen to the [MAXNG][MAXN1] shape of cell_values
   double Sn[MAXNG][MAXN1] = {};
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(CB) void k_transport_speed(OpArgs O,
   double local_max = 0.0;
   if (batch * CB + lane < O.n_cells)
     {
-      const Phys<double> M = physics<double>(O);
+      const auto M = physics<double>(O);
       const double ij[2] = {1.0 / O.hxy[((size_t)batch * 2) * CB + lane],
                             1.0 / O.hxy[((size_t)batch * 2 + 1) * CB + lane]};
       // the power iteration depends on the cell only
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(CB) void k_volume(OpArgs O, const double *__restric
   double sum = 0.0;
   if (batch * CB + lane < O.n_cells)
     {
-      const Phys<double> M = physics<double>(O);
+      const auto M = physics<double>(O);
       const double area = O.hxy[((size_t)batch * 2) * CB + lane] *
                           O.hxy[((size_t)batch * 2 + 1) * CB + lane];
       double U[ND], z[NP];

@@ -49,8 +49,8 @@ constexpr bool centred()
 }
 
 // exterior state on a boundary face (OceanDG.h:1130-1203 / 1246-1317); returns at_outflow
-template <typename T>
-__device__ __forceinline__ bool boundary_state(const Phys<T> &M, int kind, T zm, Vec2<T> qm,
+template <typename T, bool FLAT>
+__device__ __forceinline__ bool boundary_state(const Phys<T, FLAT> &M, int kind, T zm, Vec2<T> qm,
                                                Vec2<T> n, T zb, const double *bv, T &zp,
                                                Vec2<T> &qp)
 {
@@ -156,8 +156,8 @@ __device__ __forceinline__ void restrict_half(const Basis<R> &T, int half, R *z,
 
 // integral over one (sub)face of NG Gauss-Lobatto points: both traces as nodal values on
 // the (sub)face, deviations from zcr / zc2r; acc[cc][k] = sum_a Sg[a][k] inner(..)_cc JxW_a
-template <int P, int NC, typename R, typename InnerFn>
-__device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV<R> &fz, int fi,
+template <int P, int NC, typename R, bool FLAT, typename InnerFn>
+__device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV<R, FLAT> &fz, int fi,
                                                  R len, bool is_m, Vec2<R> n, const R *zo_s,
                                                  const R *xo_s, const R *yo_s, const R *zn_s,
                                                  const R *xn_s, const R *yn_s, R zcr, R zc2r,
@@ -169,9 +169,16 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
 #pragma unroll
     for (int k = 0; k < N1; ++k)
       acc[cc][k] = 0;
+  // the bed of the next point is loaded one point ahead
+  const size_t fz0 = (size_t)fi * NG * 2;
+  R zb_next[2];
+  fld_row<2, 1>(fz, fz0, zb_next);
 #pragma unroll 1
   for (int a = 0; a < NG; ++a)
     {
+      const R zbm = zb_next[0], zbp = zb_next[1];
+      if (a + 1 < NG)
+        fld_row<2, 1>(fz, fz0 + 2 * (a + 1), zb_next);
       R zo = 0, xo = 0, yo = 0, zn = 0, xn = 0, yn = 0;
 #pragma unroll
       for (int k = 0; k < N1; ++k)
@@ -186,8 +193,6 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
         }
       zo += zcr;
       zn += zc2r;
-      const R zbm = fld(fz, ((size_t)fi * NG + a) * 2 + 0);
-      const R zbp = fld(fz, ((size_t)fi * NG + a) * 2 + 1);
       R val[NC];
       inner(is_m, zo, Vec2<R>{xo, yo}, zn, Vec2<R>{xn, yn}, n, zbm, zbp, val);
       const R JxW = T.wg[a] * len;
@@ -222,9 +227,9 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
 // latency and keeps the second subface in the face loop.
 //
 // FMASK selects the faces integrated (bit f: face f); the other faces contribute nothing.
-template <int P, int NC, typename R, int FMASK = 0xF, typename ZA, typename QA, typename InnerFn,
-          typename BdryFn>
-__device__ __forceinline__ void face_terms(const OpArgs &O, const Basis<R> &T, int batch,
+template <int P, int NC, typename R, int FMASK = 0xF, typename OA, typename ZA, typename QA,
+          typename InnerFn, typename BdryFn>
+__device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int batch,
                                            int lane, R hx, R hy, const ZA &Z, const QA &QX,
                                            const QA &QY, double zc,
                                            const double *__restrict__ src_h,
@@ -287,7 +292,7 @@ __device__ __forceinline__ void face_terms(const OpArgs &O, const Basis<R> &T, i
           const int bk = O.bkind[bf];
           const Vec2<R> n = {f == 0 ? R(-1) : f == 1 ? R(1) : R(0),
                              f == 2 ? R(-1) : f == 3 ? R(1) : R(0)};
-          const FieldV<R> bz = in_vgprs<R>(O.bdryz);
+          const auto bz = in_vgprs<R>(O, O.bdryz);
           const double *bvb = stage_bvals(O);
 #pragma unroll 1
           for (int a = 0; a < NQ; ++a)
@@ -320,7 +325,7 @@ __device__ __forceinline__ void face_terms(const OpArgs &O, const Basis<R> &T, i
         {
           const bool is_m = (f & 1);  // canonical orientation: minus side owns faces 1, 3
           const Vec2<R> n = {f < 2 ? R(1) : R(0), f < 2 ? R(0) : R(1)};
-          const FieldV<R> fz = in_vgprs<R>(O.facez);
+          const auto fz = in_vgprs<R>(O, O.facez);
           // neighbour traces of the subfaces in one group of loads (the second only on the
           // coarse side, and only where it is integrated here): one memory latency per face
           phase_barrier();
@@ -390,7 +395,7 @@ __device__ __forceinline__ void face_terms(const OpArgs &O, const Basis<R> &T, i
                 }
               const R len = (kind == FK_COARSE) ? R(0.5) * flen : flen;
               R acc[NC][N1];
-              subface_integral<P, NC, R>(T, fz, fids[f][s], len, is_m, n, zo_s, xo_s, yo_s,
+              subface_integral<P, NC>(T, fz, fids[f][s], len, is_m, n, zo_s, xo_s, yo_s,
                                          zn_s, xn_s, yn_s, zcr, R(zc2[s]), inner, acc);
               // test functions of the cell's face: the transposed restriction on the
               // coarse side
@@ -497,9 +502,9 @@ __device__ __forceinline__ void face_terms(const OpArgs &O, const Basis<R> &T, i
             }
           restrict_half<N1>(T, 1, zo_s, xo_s, yo_s);
           const Vec2<R> n = {f < 2 ? R(1) : R(0), f < 2 ? R(0) : R(1)};
-          const FieldV<R> fz = in_vgprs<R>(O.facez);
+          const auto fz = in_vgprs<R>(O, O.facez);
           R acc[NC][N1];
-          subface_integral<P, NC, R>(T, fz, fi, R(0.5) * R(hsz), (f & 1) != 0, n, zo_s, xo_s,
+          subface_integral<P, NC>(T, fz, fi, R(0.5) * R(hsz), (f & 1) != 0, n, zo_s, xo_s,
                                      yo_s, zn_s, xn_s, yn_s, R(zco), R(zc2), inner, acc);
 #pragma unroll
           for (int cc = 0; cc < NC; ++cc)
@@ -629,8 +634,8 @@ __device__ __forceinline__ void tensor_inverse(const Basis<float> &T, float *U, 
 // mass: minus side -F(own, neighbour); plus side F(neighbour, own).  Selects instead of
 // branches: the face side is a constant in the per-face loop and a lane value in the
 // compacted second-subface pass
-template <typename R>
-__device__ __forceinline__ R mass_face(const Phys<R> &M, bool is_m, R zo, Vec2<R> qo, R zn,
+template <typename R, bool FLAT>
+__device__ __forceinline__ R mass_face(const Phys<R, FLAT> &M, bool is_m, R zo, Vec2<R> qo, R zn,
                                        Vec2<R> qn, Vec2<R> n, R zbm, R zbp)
 {
   const R f = M.mass_flux(is_m ? zo : zn, is_m ? zn : zo, is_m ? qo : qn, is_m ? qn : qo, n,
@@ -640,8 +645,8 @@ __device__ __forceinline__ R mass_face(const Phys<R> &M, bool is_m, R zo, Vec2<R
 
 // momentum: minus side -(F(own, nbr) + P(own, nbr; zbm, zbp)); plus side F(nbr, own) +
 // P(own, nbr; zbp, zbm)
-template <typename R>
-__device__ __forceinline__ Vec2<R> momentum_face(const Phys<R> &M, bool is_m, R zo, Vec2<R> qo,
+template <typename R, bool FLAT>
+__device__ __forceinline__ Vec2<R> momentum_face(const Phys<R, FLAT> &M, bool is_m, R zo, Vec2<R> qo,
                                                  R zn, Vec2<R> qn, Vec2<R> n, R zbm, R zbp)
 {
   const Vec2<R> F = M.adv_flux(is_m ? zo : zn, is_m ? zn : zo, is_m ? qo : qn, is_m ? qn : qo,
@@ -653,8 +658,8 @@ __device__ __forceinline__ Vec2<R> momentum_face(const Phys<R> &M, bool is_m, R 
 // boundary face: exterior state of the condition (OceanDG.h:1130-1203 / 1246-1317), mass
 // and momentum flux; the momentum flux is cut where an outflow boundary sees backflow
 // (OceanDG.h:1326-1332)
-template <typename R>
-__device__ __forceinline__ void boundary_faces(const Phys<R> &M, int bk, R zo, Vec2<R> qo,
+template <typename R, bool FLAT>
+__device__ __forceinline__ void boundary_faces(const Phys<R, FLAT> &M, int bk, R zo, Vec2<R> qo,
                                                Vec2<R> n, R zb, const double *bv, R &mass,
                                                Vec2<R> &mom)
 {
@@ -662,7 +667,7 @@ __device__ __forceinline__ void boundary_faces(const Phys<R> &M, int bk, R zo, V
   Vec2<R> qp;
   const bool at_outflow = boundary_state(M, bk, zo, qo, n, zb, bv, zp, qp);
   mass = -M.mass_flux(zo, zp, qo, qp, n, zb, zb);
-  Vec2<R> F = M.adv_flux(zo, zp, qo, qp, n, zb, zb);
+  Vec2<R> F = M.template adv_flux<true>(zo, zp, qo, qp, n, zb, zb);
   const Vec2<R> Pr = M.pres_flux(zo, zp, n, zb, zb);
   F.x += Pr.x;
   F.y += Pr.y;
@@ -671,10 +676,10 @@ __device__ __forceinline__ void boundary_faces(const Phys<R> &M, int bk, R zo, V
   mom = {-F.x, -F.y};
 }
 
-template <typename R>
+template <typename R, bool FLAT = false>
 struct MassFaces
 {
-  Phys<R> M;
+  Phys<R, FLAT> M;
   __device__ __forceinline__ void operator()(bool is_m, R zo, Vec2<R> qo, R zn, Vec2<R> qn,
                                              Vec2<R> n, R zbm, R zbp, R *val) const
   {
@@ -690,10 +695,10 @@ struct MassFaces
   }
 };
 
-template <typename R>
+template <typename R, bool FLAT = false>
 struct MomentumFaces
 {
-  Phys<R> M;
+  Phys<R, FLAT> M;
   __device__ __forceinline__ void operator()(bool is_m, R zo, Vec2<R> qo, R zn, Vec2<R> qn,
                                              Vec2<R> n, R zbm, R zbp, R *val) const
   {
@@ -714,10 +719,10 @@ struct MomentumFaces
 
 // both equations at once (val[0] mass, val[1], val[2] momentum): the traces, velocities,
 // wave speeds and reconstructed depths of a face point are formed once for the three
-template <typename R>
+template <typename R, bool FLAT = false>
 struct AllFaces
 {
-  Phys<R> M;
+  Phys<R, FLAT> M;
   __device__ __forceinline__ void operator()(bool is_m, R zo, Vec2<R> qo, R zn, Vec2<R> qn,
                                              Vec2<R> n, R zbm, R zbp, R *val) const
   {
@@ -840,10 +845,10 @@ __device__ __forceinline__ double load_own(const double *__restrict__ src_h,
   return zc;
 }
 
-template <typename R>
-__device__ __forceinline__ Phys<R> physics(const OpArgs &O)
+template <typename R, typename OA>
+__device__ __forceinline__ Phys<R, OA::FLAT> physics(const OA &O)
 {
-  return Phys<R>{R(O.g), R(O.cu4), R(O.nu)};
+  return {R(O.g), R(O.cu4), R(O.nu)};
 }
 
 // L_zeta (INVERT: M^-1 L_zeta, for apply())
@@ -859,7 +864,7 @@ __global__ __launch_bounds__(CB) void k_height_rhs(OpArgs O, const double *__res
   const int lane = threadIdx.x & (CB - 1);
   if (batch * CB + lane >= O.n_cells)
     return;
-  const Phys<R> M = physics<R>(O);
+  const auto M = physics<R>(O);
   const R hx = R(O.hxy[((size_t)batch * 2) * CB + lane]);
   const R hy = R(O.hxy[((size_t)batch * 2 + 1) * CB + lane]);
   R Z[ND], QX[ND], QY[ND];
@@ -962,8 +967,8 @@ __device__ __forceinline__ void pair_exchange(R (&A)[3][(P + 1) * (P + 1)], R *x
 // Coriolis; OceanDG.h:696-743, ShallowWater.h:381-432): AX, AY += the integrals against
 // grad(phi) and phi.  The batch's own zeta (deviation from zcr), q (and velocity) are read
 // from the lane-interleaved LDS copy `lds`.
-template <int P, bool VISC, typename R>
-__device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis<R> &T,
+template <int P, bool VISC, typename R, typename OA>
+__device__ __forceinline__ void discharge_cell_term(const OA &O, const Basis<R> &T,
                                                     const R *lds, int batch, int lane, R hx,
                                                     R hy, R zcr, R (&AX)[(P + 1) * (P + 1)],
                                                     R (&AY)[(P + 1) * (P + 1)])
@@ -971,14 +976,16 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P);
   const LdsVec<R> Z{lds + lane}, QX{lds + ND * CB + lane}, QY{lds + 2 * ND * CB + lane};
   const LdsVec<R> UX{lds + 3 * ND * CB + lane}, UY{lds + 4 * ND * CB + lane};
-  const Phys<R> M = physics<R>(O);
+  const auto M = physics<R>(O);
   const R g = R(O.g), nu = R(O.nu);
   const R ihx = R(1) / hx, ihy = R(1) / hy, area = hx * hy;
   const size_t c0base = (size_t)batch * NQ * NQ * CB + lane;
-  const FieldV<R> bed = in_vgprs<R>(O.cell0[0]);
+  const auto bed = in_vgprs<R>(O, O.cell0[0]);
 #pragma unroll 1
   for (int b = 0; b < NQ; ++b)
     {
+      R zb[NQ];
+      fld_row<NQ, CB>(bed, c0base + (size_t)NQ * b * CB, zb);
       // the own nodal values are read from LDS again in every row: hoisted out of the loop
       // they would stay live in 3 nd registers (FP64: 6 nd) across the whole cell term,
       // which held the FP64 kernels at p = 3 to one wave per SIMD
@@ -1039,8 +1046,7 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
           zy *= ihy;
           const int q = a + NQ * b;
           const size_t pi = c0base + (size_t)q * CB;
-          const R zb = fld(bed, pi);
-          const R h = M.depth(z, zb);
+          const R h = M.depth(z, zb[a]);
           const R s = M.inv_depth(h);
           const R vx = qx * s, vy = qy * s;
           R F00 = qx * vx, F01 = qx * vy, F10 = qy * vx, F11 = qy * vy;
@@ -1067,23 +1073,23 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
             }
           const R mgh = -g * h;
           R Sx = mgh * zx, Sy = mgh * zy;
-          if (O.has_friction)
+          if (O.friction())
             {
               const R n_m = R(fld(O.cell0[1], pi));
               const R hcf = manning_coefficient(g, n_m, h, vx, vy);
-              Sx -= hcf * vx;
-              Sy -= hcf * vy;
+              Sx = plus_product(Sx, -hcf, vx);
+              Sy = plus_product(Sy, -hcf, vy);
             }
-          if (O.has_wind)
+          if (O.wind())
             {
               Sx += R(fld(O.cell0[2], pi));
               Sy += R(fld(O.cell0[3], pi));
             }
-          if (O.has_coriolis)
+          if (O.coriolis())
             {
               const R fc = R(fld(O.cell0[4], pi));
-              Sx += fc * qy;
-              Sy += -fc * qx;
+              Sx = plus_product(Sx, fc, qy);
+              Sy = plus_product(Sy, -fc, qx);
             }
           const R JxW = T.wq[a] * T.wq[b] * area;
           const R g0x = F00 * ihx * JxW, g0y = F01 * ihy * JxW;
@@ -1092,9 +1098,9 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
 #pragma unroll
           for (int i = 0; i < N1; ++i)
             {
-              WSX[i] += T.Sq[a][i] * v0 + T.Dq[a][i] * g0x;
+              WSX[i] += two_products(T.Sq[a][i], v0, T.Dq[a][i], g0x);
               WDX[i] += T.Sq[a][i] * g0y;
-              WSY[i] += T.Sq[a][i] * v1 + T.Dq[a][i] * g1x;
+              WSY[i] += two_products(T.Sq[a][i], v1, T.Dq[a][i], g1x);
               WDY[i] += T.Sq[a][i] * g1y;
             }
         }
@@ -1103,16 +1109,17 @@ __device__ __forceinline__ void discharge_cell_term(const OpArgs &O, const Basis
 #pragma unroll
         for (int i = 0; i < N1; ++i)
           {
-            AX[i + N1 * j] += T.Sq[b][j] * WSX[i] + T.Dq[b][j] * WDX[i];
-            AY[i + N1 * j] += T.Sq[b][j] * WSY[i] + T.Dq[b][j] * WDY[i];
+            AX[i + N1 * j] += two_products(T.Sq[b][j], WSX[i], T.Dq[b][j], WDX[i]);
+            AY[i + N1 * j] += two_products(T.Sq[b][j], WSY[i], T.Dq[b][j], WDY[i]);
           }
     }
 }
 
 // IN32 (FP32 paired stage): the stage input S.src_h, S.src_q comes in its centred FP32 form
 // (c32_values, c32_centres); S.out32: the RK update writes the next stage input so
-template <int P, bool VISC, int MODE, typename R, bool PAIR = false, bool IN32 = false>
-__device__ __forceinline__ void discharge_block(const OpArgs &O, const StageArgs &S, int batch,
+template <int P, bool VISC, int MODE, typename R, bool PAIR = false, bool IN32 = false,
+          typename OA = OpArgs>
+__device__ __forceinline__ void discharge_block(const OA &O, const StageArgs &S, int batch,
                                                 R *lds, R *xch = nullptr)
 {
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P);
@@ -1230,7 +1237,7 @@ __device__ __forceinline__ void discharge_block(const OpArgs &O, const StageArgs
           area = hx * hy;
           discharge_cell_term<P, VISC, R>(O, T, lds, batch, lane, hx, hy, R(zc), A[1], A[2]);
           phase_barrier();
-          const AllFaces<R> fn{physics<R>(O)};
+          const AllFaces<R, OA::FLAT> fn{physics<R>(O)};
           face_terms<P, 3, R, 0xC>(O, T, batch, lane, hx, hy, Z, QX, QY, zc, src_h, src_q, A,
                                    fn, fn, IN32);
         }
@@ -1244,13 +1251,13 @@ __device__ __forceinline__ void discharge_block(const OpArgs &O, const StageArgs
   else if (active)
     {
       const LdsVec<R> Z{lds + lane}, QX{lds + ND * CB + lane}, QY{lds + 2 * ND * CB + lane};
-      const Phys<R> M = physics<R>(O);
+      const auto M = physics<R>(O);
       const R hx = R(O.hxy[((size_t)batch * 2) * CB + lane]);
       const R hy = R(O.hxy[((size_t)batch * 2 + 1) * CB + lane]);
       area = hx * hy;
       discharge_cell_term<P, VISC, R>(O, T, lds, batch, lane, hx, hy, R(zc), Racc[0], Racc[1]);
       phase_barrier();
-      const MomentumFaces<R> fn{M};
+      const MomentumFaces<R, OA::FLAT> fn{M};
       face_terms<P, 2, R>(O, T, batch, lane, hx, hy, Z, QX, QY, zc, src_h, src_q, Racc, fn, fn);
     }
   if (MODE == 2 || MODE == 4)
@@ -1382,7 +1389,7 @@ __device__ __forceinline__ int depth_mass(const OpArgs &O, const DegreeTables &T
   const size_t zbase = (size_t)batch * NG * NG * CB + lane;
   int ndry = 0;
   hmin = DBL_MAX;
-  const FieldV<double> bed = in_vgprs<double>(O.cell1);
+  const auto bed = in_vgprs<double>(O, O.cell1);
 #pragma unroll 1
   for (int b = 0; b < NG; ++b)
     {
@@ -1500,7 +1507,7 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
     const size_t zbase = (size_t)batch * NP * CB + lane;
     double zbmax = -DBL_MAX;
     int ndry = 0;
-    const FieldV<double> bed = in_vgprs<double>(O.cell1);
+    const auto bed = in_vgprs<double>(O, O.cell1);
 #pragma unroll 1
     for (int b = 0; b < NG; ++b)
       {
@@ -1612,18 +1619,19 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
 
 // least depth of zeta^n = Z at the GL(p+2) points; NaN where an entry of Z is not finite (fmin
 // drops NaN), which no cell's certificate passes
-template <int P>
-__device__ __forceinline__ double least_depth(const OpArgs &O, const DegreeTables &T, int batch,
+template <int P, typename OA>
+__device__ __forceinline__ double least_depth(const OA &O, const DegreeTables &T, int batch,
                                               int lane, const double *Z)
 {
   constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
   double hmin = DBL_MAX;
   const size_t zbase = (size_t)batch * NG * NG * CB + lane;
-  const FieldV<double> bed = in_vgprs<double>(O.cell1);
+  const auto bed = in_vgprs<double>(O, O.cell1);
 #pragma unroll 1
   for (int b = 0; b < NG; ++b)
     {
-      double zs[N1];
+      double zb[NG], zs[N1];
+      fld_row<NG, CB>(bed, zbase + (size_t)NG * b * CB, zb);
 #pragma unroll
       for (int i = 0; i < N1; ++i)
         {
@@ -1640,7 +1648,7 @@ __device__ __forceinline__ double least_depth(const OpArgs &O, const DegreeTable
 #pragma unroll
           for (int i = 0; i < N1; ++i)
             z += T.Sg[a][i] * zs[i];
-          hmin = fmin(hmin, z + fld(bed, zbase + (size_t)(a + NG * b) * CB));
+          hmin = fmin(hmin, z + zb[a]);
         }
     }
   double zsum = 0.0;
@@ -1756,8 +1764,8 @@ __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &
 }
 
 // the same for the FP32 stage: formed in FP32 on the deviation from node 0
-template <int P>
-__device__ __forceinline__ float least_depth32(const OpArgs &O, int batch, int lane,
+template <int P, typename OA>
+__device__ __forceinline__ float least_depth32(const OA &O, int batch, int lane,
                                                const double *Z)
 {
   constexpr int N1 = P + 1, ND = N1 * N1, NG = P + 2;
@@ -1769,10 +1777,12 @@ __device__ __forceinline__ float least_depth32(const OpArgs &O, int batch, int l
     dev[i] = float(Z[i] - zc);
   float hmin = FLT_MAX;
   const size_t zbase = (size_t)batch * NG * NG * CB + lane;
-  const FieldV<double> bed = in_vgprs<double>(O.cell1);
+  const auto bed = in_vgprs<double>(O, O.cell1);
 #pragma unroll 1
   for (int b = 0; b < NG; ++b)
     {
+      double zb[NG];
+      fld_row<NG, CB>(bed, zbase + (size_t)NG * b * CB, zb);
       float zs[N1];
 #pragma unroll
       for (int i = 0; i < N1; ++i)
@@ -1790,8 +1800,7 @@ __device__ __forceinline__ float least_depth32(const OpArgs &O, int batch, int l
 #pragma unroll
           for (int i = 0; i < N1; ++i)
             z += Tf.Sg[a][i] * zs[i];
-          const double zb = fld(bed, zbase + (size_t)(a + NG * b) * CB);
-          const float h = float(zc + zb) + z;
+          const float h = float(zc + zb[a]) + z;
           hmin = h < hmin ? h : hmin;
         }
     }
@@ -1922,7 +1931,7 @@ __global__ __launch_bounds__(CB) void k_height_jacobi(OpArgs O, StageArgs S)
   const int batch = logical_batch(blockIdx.x, O.n_batches, O.xcd_swizzle);
   const int lane = threadIdx.x & (CB - 1);
   const bool active = batch * CB + lane < O.n_cells;
-  const Phys<double> M = physics<double>(O);
+  const Phys<double> M = physics<double>(static_cast<const OpArgs &>(O));
   int k = 0;
   double F[ND], Z[ND], area = 1.0;
   if (active)
@@ -1982,7 +1991,7 @@ __device__ __forceinline__ void depth_deferred_batch(const OpArgs &O, const Stag
   int k = 0;
   if (mine)
     {
-      const Phys<double> M = physics<double>(O);
+      const Phys<double> M = physics<double>(static_cast<const OpArgs &>(O));
       const double hx = O.hxy[((size_t)batch * 2) * CB + lane];
       const double hy = O.hxy[((size_t)batch * 2 + 1) * CB + lane];
       const double area = hx * hy;
@@ -2049,8 +2058,9 @@ __global__ __launch_bounds__(CB) void k_depth_deferred(OpArgs O, StageArgs S)
 // registers for the front (it is also written out as ki_h[stage+1] for later stages).
 // IN32 / S.out32 as for discharge_block (the zeta register's centres included)
 // MODE 1, 2 (paired only): apply and rhs, M^-1 L_zeta or L_zeta into the FP64 vector S.dst
-template <int P, typename R, bool PAIR = false, bool IN32 = false, int MODE = 0>
-__device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageArgs &S,
+template <int P, typename R, bool PAIR = false, bool IN32 = false, int MODE = 0,
+          typename OA = OpArgs>
+__device__ __forceinline__ void height_stage_block(const OA &O, const StageArgs &S,
                                                    int batch, float *lds, R *xch = nullptr,
                                                    const R *own = nullptr)
 {
@@ -2058,7 +2068,7 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
   const DegreeTables &T = basis<double>(P);
   const int lane = threadIdx.x & (CB - 1);
   const bool active = batch * CB + lane < O.n_cells;
-  const Phys<double> M = physics<double>(O);
+  const Phys<double> M = physics<double>(static_cast<const OpArgs &>(O));
   int k = 0;
   double F[ND], Z[ND], area = 1.0;
   typename std::conditional<centred<R>(), float, double>::type hmin = 0;
@@ -2129,7 +2139,7 @@ __device__ __forceinline__ void height_stage_block(const OpArgs &O, const StageA
           const LdsVec<R> Zo{own + lane}, QX{own + ND * CB + lane}, QY{own + 2 * ND * CB + lane};
           height_cell_term<P, R>(basis<R>(P), R(hx), R(hy), QX, QY, A[0]);
           phase_barrier();
-          const AllFaces<R> fn{physics<R>(O)};
+          const AllFaces<R, OA::FLAT> fn{physics<R>(O)};
           face_terms<P, 3, R, 0x3>(O, basis<R>(P), batch, lane, R(hx), R(hy), Zo, QX, QY, zc,
                                    S.src_h, S.src_q, A, fn, fn, IN32);
         }
@@ -2330,9 +2340,11 @@ __device__ __forceinline__ bool pair_height_wave()
 // time loop's intermediate stages); a compile-time variant, so that neither form's kernel
 // carries the other's loads
 // MODE 1, 2: apply (M^-1 L) and rhs (L) of Q.src_h, Q.src_q into H.dst, Q.dst
-template <int P, typename R, bool IN32 = false, bool VISC = false, int MODE = 0>
+// OA: which terms are known at compile time (OpArgs: none)
+template <int P, typename R, bool IN32 = false, bool VISC = false, int MODE = 0,
+          typename OA = OpArgs>
 __global__ __launch_bounds__(2 * CB, (stage_min_waves<P, false, R>())) void k_stage_pair(
-  OpArgs O, StageArgs H, StageArgs Q)
+  OA O, StageArgs H, StageArgs Q)
 {
   __shared__ __align__(16) R lds[pair_lds_words<P, R, VISC>()];
   const int batch = logical_batch(blockIdx.x, O.n_batches, O.xcd_swizzle);
