@@ -49,9 +49,13 @@ __device__ __forceinline__ void stiff_source(const OpArgs &O, const Basis<R> &T,
   for (int k = 0; k < ND; ++k)
     Rx[k] = Ry[k] = 0;
   const size_t c0base = (size_t)batch * NQ * NQ * CB + lane;
+  const auto bed = in_vgprs<R>(O, O.cell0[0]), friction = in_vgprs<R>(O, O.cell0[1]);
 #pragma unroll 1
   for (int b = 0; b < NQ; ++b)
     {
+      R zb[NQ], nm[NQ];
+      fld_row<NQ, CB>(bed, c0base + (size_t)NQ * b * CB, zb);
+      fld_row<NQ, CB>(friction, c0base + (size_t)NQ * b * CB, nm);
       R zs[N1], xs[N1], ys[N1], WX[N1], WY[N1];
 #pragma unroll
       for (int i = 0; i < N1; ++i)
@@ -81,14 +85,11 @@ __device__ __forceinline__ void stiff_source(const OpArgs &O, const Basis<R> &T,
               qy += T.Sq[a][i] * ys[i];
             }
           z += zcr;
-          const size_t pi = c0base + (size_t)(a + NQ * b) * CB;
-          const R zb = R(fld(O.cell0[0], pi));
-          const R n_m = R(fld(O.cell0[1], pi));
           // ShallowWater.h:461-472, BottomFriction.h:186-199
-          const R h = M.depth(z, zb);
+          const R h = M.depth(z, zb[a]);
           const R s = M.inv_depth(h);
           const R vx = qx * s, vy = qy * s;
-          const R hcf = manning_coefficient(M.g, n_m, h, vx, vy);
+          const R hcf = manning_coefficient(M.g, nm[a], h, vx, vy);
           const R JxW = T.wq[a] * T.wq[b] * area;
           const R v0 = -(hcf * vx) * JxW, v1 = -(hcf * vy) * JxW;
 #pragma unroll
@@ -242,12 +243,18 @@ __device__ __forceinline__ void ark_update_cell(const OpArgs &O, const ArkArgs &
         U[k] = A.ri_q[vix(batch, 2, 1, ND, k, lane)];
       tensor_apply_T<P>(SnT, U, qy);
       const size_t c2 = (size_t)batch * ND * CB + lane;
+      const auto bed = in_vgprs<double>(O, O.cell2), friction = in_vgprs<double>(O, O.cell2n);
+      double zb[N1], cfr[N1];
 #pragma unroll
       for (int k = 0; k < ND; ++k)
         {
-          const double zb = fld(O.cell2, c2 + (size_t)k * CB);
-          const double cf = fld(O.cell2n, c2 + (size_t)k * CB);
-          const double h = M.depth(z[k], zb);
+          if (k % N1 == 0)
+            {
+              fld_row<N1, CB>(bed, c2 + (size_t)k * CB, zb);
+              fld_row<N1, CB>(friction, c2 + (size_t)k * CB, cfr);
+            }
+          const double cf = cfr[k % N1];
+          const double h = M.depth(z[k], zb[k % N1]);
           const double s = M.inv_depth(h);
           const double vx = qx[k] * s, vy = qy[k] * s;
           // BottomFrictionManning::jacobian (BottomFriction.h:201-212)
@@ -345,8 +352,8 @@ __global__ __launch_bounds__(CB) void k_ark_update(OpArgs O, ArkArgs A)
 // input (read from the LDS copy of the batch's own data, still intact) stored as kim; then
 // the modified-mass update of each cell (ark_update_cell, which reads this stage's kex and
 // kim back from the vectors this lane has just written).
-template <int P, typename R>
-__device__ __forceinline__ void discharge_ark_block(const OpArgs &O, const StageArgs &Q,
+template <int P, typename R, typename OA>
+__device__ __forceinline__ void discharge_ark_block(const OA &O, const StageArgs &Q,
                                                     const ArkArgs &A, int batch, R *lds,
                                                     R *xch)
 {
@@ -362,7 +369,8 @@ __device__ __forceinline__ void discharge_ark_block(const OpArgs &O, const Stage
       const double zc = centred<R>() ? Q.src_h[vix(batch, 1, 0, ND, 0, lane)] : 0.0;
       const LdsVec<R> Z{lds + lane}, QX{lds + ND * CB + lane}, QY{lds + 2 * ND * CB + lane};
       R Rx[ND], Ry[ND];
-      stiff_source<P, R>(O, basis<R>(P), Z, QX, QY, R(zc), batch, lane, hx * hy, Rx, Ry);
+      stiff_source<P, R>(static_cast<const OpArgs &>(O), basis<R>(P), Z, QX, QY, R(zc), batch, lane,
+                         hx * hy, Rx, Ry);
       R *kim = reinterpret_cast<R *>(A.kim_out);
 #pragma unroll
       for (int k = 0; k < ND; ++k)
@@ -390,9 +398,9 @@ constexpr int ark_min_waves()
   return std::is_same<R, float>::value ? (P <= 2 ? 3 : P == 3 ? 2 : 1) : (P <= 3 ? 2 : 1);
 }
 
-template <int P, typename R>
+template <int P, typename R, typename OA>
 __global__ __launch_bounds__(2 * CB, (ark_min_waves<P, R>())) void k_stage_ark_pair(
-  OpArgs O, StageArgs H, StageArgs Q, ArkArgs A)
+  OA O, StageArgs H, StageArgs Q, ArkArgs A)
 {
   __shared__ __align__(16) R lds[pair_lds_words<P, R>()];
   const int batch = logical_batch(blockIdx.x, O.n_batches, O.xcd_swizzle);
@@ -456,7 +464,16 @@ int launch_stage_ark(oc_dg *op, const OpArgs &O, uint32_t stage, uint32_t n_stag
       A.wq_out = w_q;
       A.kim_out = last ? nullptr : ki_q[2 * stage + 2];
       timed_begin(op, s, &ev);
-      hipLaunchKernelGGL((k_stage_ark_pair<P, R>), grid, dim3(2 * CB), 0, s, Oe, H, Q, A);
+      auto launch = [&](auto args) {
+        hipLaunchKernelGGL((k_stage_ark_pair<P, R, decltype(args)>), grid, dim3(2 * CB), 0, s, args,
+                           H, Q, A);
+      };
+      if (is_bare(Oe))
+        launch(BareArgs{Oe});
+      else if (is_manning(Oe))
+        launch(ManningArgs{Oe});
+      else
+        launch(Oe);
       timed_end(op, s, TK_STAGE, ev);
       HIP_TRY(hipGetLastError());
       if (std::is_same<R, float>::value && defer_depth_solve(P))

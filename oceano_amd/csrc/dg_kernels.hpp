@@ -29,7 +29,6 @@ struct Basis
   R Dq[MAXNQ][MAXN1];      // l_i' at Gauss(nq) points
   R wq[MAXNQ];
   R Sg[MAXNG][MAXN1];      // l_i at Gauss-Lobatto(ng) points
-  R Sgs[2][MAXNG][MAXN1];  // l_i at (t + s)/2, t in GL(ng): coarse side of subface s
   R wg[MAXNG];
   R Ti[MAXN1][MAXN1];      // inverse of [l_i(Gauss(n1)_a)]_{a,i}, stored [i][a]
   R wn[MAXN1];             // Gauss(n1) weights
@@ -112,8 +111,12 @@ struct OpArgs
 // then cannot be interleaved, and with one to three waves per SIMD each point waits out its own
 // chain of dependent instructions.  RK4 step of 97,280 cells at p = 3 mixed 177 -> 159 us, FP64
 // 355 -> 320 us; of 12,800 at p = 1 FP64 40 -> 35 us; channel of 2,500 at p = 2 FP64 79 -> 70 us.
+// In the other kernels: M^-1 L of 25,538 cells at p = 4 FP64 56 -> 45 us, viscous RK4 step of
+// 51,200 at p = 2 130 -> 119 us, RK4 step of a twelve-instance ensemble of p = 1 to 4 mixed 237 -> 210 us, additive step of 64,464
+// channel cells at p = 2 155 -> 149 us.
 //   PlainArgs    no friction, wind or Coriolis force, every bed field uniform
 //   ManningArgs  friction, neither wind nor Coriolis force, any bed
+//   BareArgs     none of the three, any bed (the explicit part of the additive stage)
 struct PlainArgs : OpArgs
 {
   static constexpr bool FLAT = true;
@@ -127,6 +130,12 @@ struct ManningArgs : OpArgs
   __host__ __device__ static constexpr bool wind() { return false; }
   __host__ __device__ static constexpr bool coriolis() { return false; }
 };
+struct BareArgs : OpArgs
+{
+  __host__ __device__ static constexpr bool friction() { return false; }
+  __host__ __device__ static constexpr bool wind() { return false; }
+  __host__ __device__ static constexpr bool coriolis() { return false; }
+};
 inline bool is_plain(const OpArgs &O)
 {
   return !O.has_friction && !O.has_wind && !O.has_coriolis && !O.cell0[0].ptr && !O.cell1.ptr &&
@@ -135,6 +144,10 @@ inline bool is_plain(const OpArgs &O)
 inline bool is_manning(const OpArgs &O)
 {
   return O.has_friction && !O.has_wind && !O.has_coriolis;
+}
+inline bool is_bare(const OpArgs &O)
+{
+  return !O.has_friction && !O.has_wind && !O.has_coriolis;
 }
 
 struct StageArgs

@@ -76,6 +76,18 @@ inline void stage_args(const OpArgs &O, uint32_t stage, const double *factor,
   H.sweeps_blk = O.sweeps;
 }
 
+// launch(args) with the argument type that says which terms there are
+template <typename Fn>
+inline void with_terms(const OpArgs &O, Fn launch)
+{
+  if (is_plain(O))
+    launch(PlainArgs{O});
+  else if (is_manning(O))
+    launch(ManningArgs{O});
+  else
+    launch(O);
+}
+
 template <int P, typename R>
 int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *factor,
                  const double *ri_h, const double *ri_q, const double *ri_v,
@@ -105,7 +117,10 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
           // waves' registers and the unpaired items at one wave per SIMD are faster (26,000 hanging
           // cells at p = 3: 196 us a step, paired 225; 5,000 at p = 4: 264, paired 279)
           if constexpr (std::is_same<R, double>::value && P <= 2)
-            hipLaunchKernelGGL((k_stage_pair<P, R, false, true>), grid, dim3(2 * CB), 0, s, O, H, Q);
+            with_terms(O, [&](auto args) {
+              hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 0, decltype(args)>), grid,
+                                 dim3(2 * CB), 0, s, args, H, Q);
+            });
           else
             hipLaunchKernelGGL((k_stage<P, true, R, 1>), dim3(items), block, 0, s, O, H, Q);
         }
@@ -114,7 +129,7 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
           constexpr bool C32 = std::is_same<R, float>::value && P <= 3;
           if (C32)
             H.out32 = Q.out32 = op->rk_out32 && !last;
-          auto launch = [&](auto args) {
+          with_terms(O, [&](auto args) {
             using OA = decltype(args);
             if (C32 && op->rk_in32)
               hipLaunchKernelGGL((k_stage_pair<P, R, C32, false, 0, OA>), grid, dim3(2 * CB), 0, s,
@@ -122,22 +137,20 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
             else
               hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 0, OA>), grid, dim3(2 * CB), 0,
                                  s, args, H, Q);
-          };
-          if (is_plain(O))
-            launch(PlainArgs{O});
-          else if (is_manning(O))
-            launch(ManningArgs{O});
-          else
-            launch(O);
+          });
         }
-      else if (op->waves_per_block == 4)
-        hipLaunchKernelGGL((k_stage<P, false, R, 4>), dim3((items + 3) / 4), dim3(4 * CB), 0,
-                           s, O, H, Q);
-      else if (op->waves_per_block == 2)
-        hipLaunchKernelGGL((k_stage<P, false, R, 2>), dim3((items + 1) / 2), dim3(2 * CB), 0,
-                           s, O, H, Q);
       else
-        hipLaunchKernelGGL((k_stage<P, false, R, 1>), dim3(items), block, 0, s, O, H, Q);
+        with_terms(O, [&](auto args) {
+          using OA = decltype(args);
+          if (op->waves_per_block == 4)
+            hipLaunchKernelGGL((k_stage<P, false, R, 4, OA>), dim3((items + 3) / 4), dim3(4 * CB),
+                               0, s, args, H, Q);
+          else if (op->waves_per_block == 2)
+            hipLaunchKernelGGL((k_stage<P, false, R, 2, OA>), dim3((items + 1) / 2), dim3(2 * CB),
+                               0, s, args, H, Q);
+          else
+            hipLaunchKernelGGL((k_stage<P, false, R, 1, OA>), dim3(items), block, 0, s, args, H, Q);
+        });
       timed_end(op, s, TK_STAGE, ev);
       HIP_TRY(hipGetLastError());
       if (std::is_same<R, float>::value && defer_depth_solve(P))
@@ -211,27 +224,38 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
       const dim3 pair(2 * CB);
       if (invert && visc)
         hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 1>), grid, pair, 0, s, O, H, S);
-      else if (invert)
-        hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 1>), grid, pair, 0, s, O, H, S);
       else if (visc)
         hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 2>), grid, pair, 0, s, O, H, S);
       else
-        hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 2>), grid, pair, 0, s, O, H, S);
+        with_terms(O, [&](auto args) {
+          using OA = decltype(args);
+          if (invert)
+            hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 1, OA>), grid, pair, 0, s, args,
+                               H, S);
+          else
+            hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 2, OA>), grid, pair, 0, s, args,
+                               H, S);
+        });
     }
   else
     {
-      if (invert)
-        hipLaunchKernelGGL((k_height_rhs<P, true, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
-      else
-        hipLaunchKernelGGL((k_height_rhs<P, false, R>), grid, block, 0, s, O, src_h, src_q, dst_h);
+      with_terms(O, [&](auto args) {
+        using OA = decltype(args);
+        if (invert)
+          hipLaunchKernelGGL((k_height_rhs<P, true, R, double, OA>), grid, block, 0, s, args, src_h,
+                             src_q, dst_h);
+        else
+          hipLaunchKernelGGL((k_height_rhs<P, false, R, double, OA>), grid, block, 0, s, args, src_h,
+                             src_q, dst_h);
+        if (invert && !visc)
+          hipLaunchKernelGGL((k_discharge<P, false, 1, R, OA>), grid, block, 0, s, args, S);
+        else if (!visc)
+          hipLaunchKernelGGL((k_discharge<P, false, 2, R, OA>), grid, block, 0, s, args, S);
+      });
       if (invert && visc)
         hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
-      else if (invert)
-        hipLaunchKernelGGL((k_discharge<P, false, 1, R>), grid, block, 0, s, O, S);
       else if (visc)
         hipLaunchKernelGGL((k_discharge<P, true, 2, R>), grid, block, 0, s, O, S);
-      else
-        hipLaunchKernelGGL((k_discharge<P, false, 2, R>), grid, block, 0, s, O, S);
     }
   HIP_TRY(hipGetLastError());
   return OC_OK;

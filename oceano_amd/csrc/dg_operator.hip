@@ -104,11 +104,7 @@ DegreeTables make_tables(int p)
     {
       t.wg[a] = rg.w[a];
       for (int i = 0; i < n1; ++i)
-        {
-          t.Sg[a][i] = lagrange_value(nodes.x, i, rg.x[a]);
-          for (int s = 0; s < 2; ++s)
-            t.Sgs[s][a][i] = lagrange_value(nodes.x, i, 0.5 * (rg.x[a] + s));
-        }
+        t.Sg[a][i] = lagrange_value(nodes.x, i, rg.x[a]);
     }
   std::vector<double> S(n1 * n1);
   for (int a = 0; a < n1; ++a)

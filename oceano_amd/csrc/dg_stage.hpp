@@ -800,9 +800,9 @@ __device__ __forceinline__ void height_cell_term(const Basis<R> &T, R hx, R hy, 
 // ---------------------------------------------------------------------------------------
 // L_zeta of one cell (cell term + faces) into Racc
 // ---------------------------------------------------------------------------------------
-template <int P, typename R, typename ZA, typename QA>
-__device__ __forceinline__ void height_operator(const OpArgs &O, const Basis<R> &T,
-                                                const Phys<R> &M, int batch, int lane, R hx,
+template <int P, typename R, typename OA, typename ZA, typename QA>
+__device__ __forceinline__ void height_operator(const OA &O, const Basis<R> &T,
+                                                const Phys<R, OA::FLAT> &M, int batch, int lane, R hx,
                                                 R hy, const ZA &Z, const QA &QX, const QA &QY,
                                                 double zc, const double *__restrict__ src_h,
                                                 const double *__restrict__ src_q,
@@ -814,7 +814,7 @@ __device__ __forceinline__ void height_operator(const OpArgs &O, const Basis<R> 
     Racc[0][k] = 0;
   height_cell_term<P, R>(T, hx, hy, QX, QY, Racc[0]);
   phase_barrier();
-  const MassFaces<R> fn{M};
+  const MassFaces<R, OA::FLAT> fn{M};
   face_terms<P, 1, R>(O, T, batch, lane, hx, hy, Z, QX, QY, zc, src_h, src_q, Racc, fn, fn);
 }
 
@@ -853,8 +853,8 @@ __device__ __forceinline__ Phys<R, OA::FLAT> physics(const OA &O)
 
 // L_zeta (INVERT: M^-1 L_zeta, for apply())
 // KT: storage type of dst (a stage's k vector is stored in R, a caller vector in FP64)
-template <int P, bool INVERT, typename R, typename KT = double>
-__global__ __launch_bounds__(CB) void k_height_rhs(OpArgs O, const double *__restrict__ src_h,
+template <int P, bool INVERT, typename R, typename KT = double, typename OA = OpArgs>
+__global__ __launch_bounds__(CB) void k_height_rhs(OA O, const double *__restrict__ src_h,
                                                    const double *__restrict__ src_q,
                                                    double *__restrict__ dst)
 {
@@ -1367,8 +1367,8 @@ __device__ __forceinline__ void discharge_block(const OA &O, const StageArgs &S,
     }
 }
 
-template <int P, bool VISC, int MODE, typename R>
-__global__ __launch_bounds__(CB) void k_discharge(OpArgs O, StageArgs S)
+template <int P, bool VISC, int MODE, typename R, typename OA = OpArgs>
+__global__ __launch_bounds__(CB) void k_discharge(OA O, StageArgs S)
 {
   __shared__ R lds[discharge_lds_words<P, VISC>()];
   discharge_block<P, VISC, MODE, R>(
@@ -2272,9 +2272,9 @@ __host__ __device__ constexpr int height_lds_words()
 // slice followed by a discharge slice, each of its own size (mixed p = 4, WPB = 2: 29 KiB per
 // workgroup, five per CU, against 38 KiB and four with two discharge-sized slices).  With
 // WPB = 1 each workgroup holds one discharge-sized slice, whatever kind its item is.
-template <int P, bool VISC, typename R, int WPB>
+template <int P, bool VISC, typename R, int WPB, typename OA = OpArgs>
 __global__ __launch_bounds__(CB * WPB, (stage_min_waves<P, VISC, R>())) void k_stage(
-  OpArgs O, StageArgs H, StageArgs Q)
+  OA O, StageArgs H, StageArgs Q)
 {
   constexpr int HW = height_lds_words<P, R>(), DW = discharge_lds_words<P, VISC>();
   __shared__ __align__(16) R lds[WPB == 1 ? DW : (WPB / 2) * (HW + DW)];

@@ -42,8 +42,8 @@ __global__ __launch_bounds__(256) void k_put_multi_args(MultiArgs A, MultiArgs *
     to[i] = src[i];
 }
 
-template <int P, typename R>
-__device__ __forceinline__ void multi_item(const OpArgs &O, const StageArgs &H,
+template <int P, typename R, typename OA>
+__device__ __forceinline__ void multi_item(const OA &O, const StageArgs &H,
                                            const StageArgs &Q, int w, R *lds)
 {
   if (item_kind(w))
@@ -58,7 +58,7 @@ constexpr int multi_min_waves()
   return stage_min_waves<4, false, R>();
 }
 
-template <typename R>
+template <typename R, typename OA>
 __global__ __launch_bounds__(CB, (multi_min_waves<R>())) void k_stage_multi(
   const MultiArgs *__restrict__ A)
 {
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(CB, (multi_min_waves<R>())) void k_stage_multi(
   int g = 0;
   while (g + 1 < A->n_groups && b >= A->start[g + 1])
     ++g;
-  const OpArgs &O = A->O[g];
+  const OA &O = static_cast<const OA &>(A->O[g]);  // the same members
   const int n_items = 2 * O.n_batches;
   const int local = b - A->start[g];
   if (local >= n_items)  // padding of the group's range to a multiple of the XCD count
@@ -94,8 +94,8 @@ __global__ __launch_bounds__(CB, (multi_min_waves<R>())) void k_stage_multi(
 // the other its discharge item (pair_height_wave); the LDS is laid out as k_stage_pair's at degree 4 (the height
 // slice of degree 4 is the largest, so every degree's height slice fits in front of the
 // discharge slice)
-template <int P, typename R>
-__device__ __forceinline__ void multi_pair(const OpArgs &O, const StageArgs &H,
+template <int P, typename R, typename OA>
+__device__ __forceinline__ void multi_pair(const OA &O, const StageArgs &H,
                                            const StageArgs &Q, int batch, R *lds)
 {
   static_assert(pair_height_words<P, R>() <= pair_height_words<4, R>() &&
@@ -109,7 +109,7 @@ __device__ __forceinline__ void multi_pair(const OpArgs &O, const StageArgs &H,
     discharge_block<P, false, 0, R, true>(O, Q, batch, dlds, xch);
 }
 
-template <typename R>
+template <typename R, typename OA>
 __global__ __launch_bounds__(2 * CB, (multi_min_waves<R>())) void k_stage_multi_pair(
   const MultiArgs *__restrict__ A)
 {
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(2 * CB, (multi_min_waves<R>())) void k_stage_multi_
   int g = 0;
   while (g + 1 < A->n_groups && b >= A->start[g + 1])
     ++g;
-  const OpArgs &O = A->O[g];
+  const OA &O = static_cast<const OA &>(A->O[g]);  // the same members
   const int local = b - A->start[g];
   if (local >= O.n_batches)  // padding of the group's range to a multiple of the XCD count
     return;
@@ -182,14 +182,25 @@ int stage_multi(int n, oc_dg *const *ops, const OpArgs *O, uint32_t stage,
   MultiArgs *dA = ops[0]->d_multi_args;
   hipLaunchKernelGGL(k_put_multi_args, dim3(1), dim3(256), 0, s, A, dA);
   HIP_TRY(hipGetLastError());
-  if (paired && mixed)
-    hipLaunchKernelGGL(k_stage_multi_pair<float>, dim3(start), dim3(2 * CB), 0, s, dA);
-  else if (paired)
-    hipLaunchKernelGGL(k_stage_multi_pair<double>, dim3(start), dim3(2 * CB), 0, s, dA);
-  else if (mixed)
-    hipLaunchKernelGGL(k_stage_multi<float>, dim3(start), dim3(CB), 0, s, dA);
+  // the groups share a kernel: flat and free of sources only if all of them are
+  bool plain = true;
+  for (int g = 0; g < n; ++g)
+    plain = plain && is_plain(O[g]);
+  auto launch = [&](auto args) {
+    using OA = decltype(args);
+    if (paired && mixed)
+      hipLaunchKernelGGL((k_stage_multi_pair<float, OA>), dim3(start), dim3(2 * CB), 0, s, dA);
+    else if (paired)
+      hipLaunchKernelGGL((k_stage_multi_pair<double, OA>), dim3(start), dim3(2 * CB), 0, s, dA);
+    else if (mixed)
+      hipLaunchKernelGGL((k_stage_multi<float, OA>), dim3(start), dim3(CB), 0, s, dA);
+    else
+      hipLaunchKernelGGL((k_stage_multi<double, OA>), dim3(start), dim3(CB), 0, s, dA);
+  };
+  if (plain)
+    launch(PlainArgs{});
   else
-    hipLaunchKernelGGL(k_stage_multi<double>, dim3(start), dim3(CB), 0, s, dA);
+    launch(OpArgs{});
   HIP_TRY(hipGetLastError());
   if (mixed)
     for (int g = 0; g < n; ++g)
