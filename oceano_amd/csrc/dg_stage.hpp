@@ -169,11 +169,15 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
 #pragma unroll
     for (int k = 0; k < N1; ++k)
       acc[cc][k] = 0;
+  // two points per trip fill each other's waits; p = 4 has no registers for it (M^-1 L of 25,538
+  // cells FP64 45.3 -> 46.5 us).  RK4 step of 97,280 cells at p = 3 FP64 321 -> 314 us, channel of
+  // 2,500 at p = 2 70.5 -> 69 us, viscous of 51,200 at p = 2 119 -> 116 us
+  constexpr int POINTS = P <= 3 ? 2 : 1;
   // the bed of the next point is loaded one point ahead
   const size_t fz0 = (size_t)fi * NG * 2;
   R zb_next[2];
   fld_row<2, 1>(fz, fz0, zb_next);
-#pragma unroll 1
+#pragma unroll POINTS
   for (int a = 0; a < NG; ++a)
     {
       const R zbm = zb_next[0], zbp = zb_next[1];
@@ -240,6 +244,9 @@ __device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int b
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P), NG = P + 2;
   constexpr bool COMPACT = std::is_same<R, float>::value;
   constexpr int NS = COMPACT ? 1 : 2;  // subfaces integrated in the face loop
+  // FP64 at p = 4: 256 registers do not hold both subfaces' traces (M^-1 L: 318 with both, 288 one
+  // by one; 46.5 us of 25,538 cells either way)
+  constexpr bool ONE_BY_ONE = NS == 2 && P >= 4;
   const R zcr = R(zc);
   // stage input in its centred FP32 form (FP32 stage only; c32_values, c32_centres)
   const bool c32 = centred<R>() && in32;
@@ -331,38 +338,38 @@ __device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int b
           phase_barrier();
           // zsub: what is subtracted from zg to centre it (0 when it comes centred)
           double zg[NS][N1], xg[NS][N1], yg[NS][N1], zc2[NS], zsub[NS];
-#pragma unroll
-          for (int s = 0; s < NS; ++s)
-            if (s == 0 || kind == FK_COARSE)
+          auto load_traces = [&](int s) {
+            const int b2 = nbrs[f][s] / CB, l2 = nbrs[f][s] % CB;
+            if (c32)
               {
-                const int b2 = nbrs[f][s] / CB, l2 = nbrs[f][s] % CB;
-                if (c32)
-                  {
-                    zc2[s] = zcen[(size_t)b2 * CB + l2];
-                    zsub[s] = 0.0;
+                zc2[s] = zcen[(size_t)b2 * CB + l2];
+                zsub[s] = 0.0;
 #pragma unroll
-                    for (int k = 0; k < N1; ++k)
-                      {
-                        const int d = face_dof<N1>(f ^ 1, k);
-                        zg[s][k] = fh[vix(b2, 1, 0, ND, d, l2)];
-                        xg[s][k] = fq[vix(b2, 2, 0, ND, d, l2)];
-                        yg[s][k] = fq[vix(b2, 2, 1, ND, d, l2)];
-                      }
-                  }
-                else
+                for (int k = 0; k < N1; ++k)
                   {
-                    zc2[s] = centred<R>() ? src_h[vix(b2, 1, 0, ND, 0, l2)] : 0.0;
-                    zsub[s] = zc2[s];
-#pragma unroll
-                    for (int k = 0; k < N1; ++k)
-                      {
-                        const int d = face_dof<N1>(f ^ 1, k);
-                        zg[s][k] = src_h[vix(b2, 1, 0, ND, d, l2)];
-                        xg[s][k] = src_q[vix(b2, 2, 0, ND, d, l2)];
-                        yg[s][k] = src_q[vix(b2, 2, 1, ND, d, l2)];
-                      }
+                    const int d = face_dof<N1>(f ^ 1, k);
+                    zg[s][k] = fh[vix(b2, 1, 0, ND, d, l2)];
+                    xg[s][k] = fq[vix(b2, 2, 0, ND, d, l2)];
+                    yg[s][k] = fq[vix(b2, 2, 1, ND, d, l2)];
                   }
               }
+            else
+              {
+                zc2[s] = centred<R>() ? src_h[vix(b2, 1, 0, ND, 0, l2)] : 0.0;
+                zsub[s] = zc2[s];
+#pragma unroll
+                for (int k = 0; k < N1; ++k)
+                  {
+                    const int d = face_dof<N1>(f ^ 1, k);
+                    zg[s][k] = src_h[vix(b2, 1, 0, ND, d, l2)];
+                    xg[s][k] = src_q[vix(b2, 2, 0, ND, d, l2)];
+                    yg[s][k] = src_q[vix(b2, 2, 1, ND, d, l2)];
+                  }
+              }
+          };
+          load_traces(0);
+          if (NS == 2 && !ONE_BY_ONE && kind == FK_COARSE)
+            load_traces(NS - 1);
           issue_barrier();
 #pragma unroll
           for (int s = 0; s < NS; ++s)
@@ -370,6 +377,11 @@ __device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int b
               if (s == 1 && kind != FK_COARSE)
                 break;
               phase_barrier();
+              if (s == 1 && ONE_BY_ONE)
+                {
+                  load_traces(s);
+                  issue_barrier();
+                }
               // both traces as nodal values on this (sub)face: the coarse side restricts
               // its own trace to half s, the fine side the neighbour's to half nsub, so
               // that every face point uses the one (wave-uniform) table Sg
