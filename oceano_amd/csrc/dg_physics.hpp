@@ -26,16 +26,17 @@ struct Vec2
 };
 
 // 1/sqrt(x) for x > 0 (the depth floor keeps every argument positive): the hardware
-// reciprocal square root refined by two Newton-Raphson steps y <- y + y (1 - x y^2) / 2,
-// within a few ulp of the correctly rounded 1/sqrt(x).  FP64: this replaces a correctly
-// rounded sqrt and a division (two multi-instruction sequences) by ~10 instructions.
+// reciprocal square root (relative error at most 5.3e-8) and one third-order step
+// y (1 + e / 2 + 3 e^2 / 8), e = 1 - x y^2.  Over 2^20 arguments in [1, 4] and [1e-40, 1e20] the
+// error is at most 1.37e-16 (rms 5.4e-17), as with the two Newton-Raphson steps that it
+// replaces (1.38e-16), in five instructions, four of them in a chain, for eight, six in a
+// chain.  RK4 step of 2,500 channel cells at p = 2 FP64 69 -> 66.5 us, of 97,280 at p = 3 314 ->
+// 311 us, additive step of 64,464 148 -> 145 us.
 __device__ __forceinline__ double rsqrt_nr(double x)
 {
-  double y = __builtin_amdgcn_rsq(x);
-  double r = __builtin_fma(-(x * y), y, 1.0);
-  y = __builtin_fma(0.5 * y, r, y);
-  r = __builtin_fma(-(x * y), y, 1.0);
-  return __builtin_fma(0.5 * y, r, y);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
 }
 // FP32 (mixed path): the hardware reciprocal square root (within 1 ulp), unrefined
 __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsqf(x); }
