@@ -215,47 +215,61 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
   S.src_q = src_q;
   S.src_v = src_v;
   S.dst = dst_q;
-  if constexpr (std::is_same<R, double>::value)
-    {
-      // one launch of paired items.  The FP32 integrals keep two launches: their results carry
-      // the order of summation of the unpaired items
-      StageArgs H = S;
-      H.dst = dst_h;
-      const dim3 pair(2 * CB);
-      if (invert && visc)
-        hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 1>), grid, pair, 0, s, O, H, S);
-      else if (visc)
-        hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 2>), grid, pair, 0, s, O, H, S);
-      else
-        with_terms(O, [&](auto args) {
-          using OA = decltype(args);
+  // FP64: one launch of paired items where its registers allow (p <= 3, viscous p <= 2).  Past that
+  // its waves need more than the 256 registers that hold both equations' integrals (p = 4: 288 to
+  // 318, viscous 378): then, and for the FP32 integrals, whose results carry the order of summation
+  // of the unpaired items, one launch for each equation.
+  constexpr bool PAIRED = std::is_same<R, double>::value && P <= 3;
+  constexpr bool PAIRED_VISC = std::is_same<R, double>::value && P <= 2;
+  StageArgs H = S;
+  H.dst = dst_h;
+  const dim3 pair(2 * CB);
+  with_terms(O, [&](auto args) {
+    using OA = decltype(args);
+    if constexpr (PAIRED)
+      if (!visc)
+        {
           if (invert)
             hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 1, OA>), grid, pair, 0, s, args,
                                H, S);
           else
             hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 2, OA>), grid, pair, 0, s, args,
                                H, S);
-        });
-    }
-  else
-    {
-      with_terms(O, [&](auto args) {
-        using OA = decltype(args);
+        }
+    if (visc ? !PAIRED_VISC : !PAIRED)
+      {
         if (invert)
           hipLaunchKernelGGL((k_height_rhs<P, true, R, double, OA>), grid, block, 0, s, args, src_h,
                              src_q, dst_h);
         else
           hipLaunchKernelGGL((k_height_rhs<P, false, R, double, OA>), grid, block, 0, s, args, src_h,
                              src_q, dst_h);
-        if (invert && !visc)
-          hipLaunchKernelGGL((k_discharge<P, false, 1, R, OA>), grid, block, 0, s, args, S);
-        else if (!visc)
-          hipLaunchKernelGGL((k_discharge<P, false, 2, R, OA>), grid, block, 0, s, args, S);
-      });
-      if (invert && visc)
-        hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
-      else if (visc)
-        hipLaunchKernelGGL((k_discharge<P, true, 2, R>), grid, block, 0, s, O, S);
+      }
+    if constexpr (!PAIRED)
+      if (!visc)
+        {
+          if (invert)
+            hipLaunchKernelGGL((k_discharge<P, false, 1, R, OA>), grid, block, 0, s, args, S);
+          else
+            hipLaunchKernelGGL((k_discharge<P, false, 2, R, OA>), grid, block, 0, s, args, S);
+        }
+  });
+  if (visc)
+    {
+      if constexpr (PAIRED_VISC)
+        {
+          if (invert)
+            hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 1>), grid, pair, 0, s, O, H, S);
+          else
+            hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 2>), grid, pair, 0, s, O, H, S);
+        }
+      else
+        {
+          if (invert)
+            hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
+          else
+            hipLaunchKernelGGL((k_discharge<P, true, 2, R>), grid, block, 0, s, O, S);
+        }
     }
   HIP_TRY(hipGetLastError());
   return OC_OK;
