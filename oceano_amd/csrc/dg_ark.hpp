@@ -491,7 +491,7 @@ int launch_stage_ark(oc_dg *op, const OpArgs &O, uint32_t stage, uint32_t n_stag
       return OC_OK;
     }
   timed_begin(op, s, &ev);
-  hipLaunchKernelGGL((k_height_rhs<P, false, R, R>), grid, block, 0, s, O, ri_h, ri_q,
+  hipLaunchKernelGGL((k_height_rhs<P, R>), grid, block, 0, s, O, ri_h, ri_q,
                      ki_h[stage + 1]);
   timed_end(op, s, TK_HEIGHT_RHS, ev);
   // explicit momentum integrals: the full operator at the last stage, without the friction

@@ -111,9 +111,9 @@ struct OpArgs
 // then cannot be interleaved, and with one to three waves per SIMD each point waits out its own
 // chain of dependent instructions.  RK4 step of 97,280 cells at p = 3 mixed 177 -> 159 us, FP64
 // 355 -> 320 us; of 12,800 at p = 1 FP64 40 -> 35 us; channel of 2,500 at p = 2 FP64 79 -> 70 us.
-// In the other kernels: M^-1 L of 25,538 cells at p = 4 FP64 56 -> 45 us, viscous RK4 step of
-// 51,200 at p = 2 130 -> 119 us, RK4 step of a twelve-instance ensemble of p = 1 to 4 mixed 237 -> 210 us, additive step of 64,464
-// channel cells at p = 2 155 -> 149 us.
+// In the other kernels: viscous RK4 step of 51,200 at p = 2 130 -> 119 us, RK4 step of a
+// twelve-instance ensemble of p = 1 to 4 mixed 237 -> 205 us, additive step of 64,464 channel
+// cells at p = 2 155 -> 149 us.
 //   PlainArgs    no friction, wind or Coriolis force, every bed field uniform
 //   ManningArgs  friction, neither wind nor Coriolis force, any bed
 //   BareArgs     none of the three, any bed (the explicit part of the additive stage)

@@ -170,7 +170,7 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
     }
   // split path: every kernel finishes reading ri before the next one overwrites it
   timed_begin(op, s, &ev);
-  hipLaunchKernelGGL((k_height_rhs<P, false, R, R>), grid, block, 0, s, O, ri_h, ri_q,
+  hipLaunchKernelGGL((k_height_rhs<P, R>), grid, block, 0, s, O, ri_h, ri_q,
                      ki_h[stage + 1]);
   timed_end(op, s, TK_HEIGHT_RHS, ev);
   timed_begin(op, s, &ev);
@@ -218,12 +218,13 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
   // FP64: one launch of paired items where its registers allow (p <= 3, viscous p <= 2).  Past that
   // its waves need more than the 256 registers that hold both equations' integrals (p = 4: 288 to
   // 318, viscous 378): then, and for the FP32 integrals, whose results carry the order of summation
-  // of the unpaired items, one launch for each equation.
+  // of the unpaired items, one launch of unpaired items. M^-1 L of 25,538 cells at p = 4 52 us
+  // (two launches, one an equation, 77; paired 46.5).
   constexpr bool PAIRED = std::is_same<R, double>::value && P <= 3;
   constexpr bool PAIRED_VISC = std::is_same<R, double>::value && P <= 2;
   StageArgs H = S;
   H.dst = dst_h;
-  const dim3 pair(2 * CB);
+  const dim3 pair(2 * CB), items(2 * op->NB);
   with_terms(O, [&](auto args) {
     using OA = decltype(args);
     if constexpr (PAIRED)
@@ -236,22 +237,13 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
             hipLaunchKernelGGL((k_stage_pair<P, R, false, false, 2, OA>), grid, pair, 0, s, args,
                                H, S);
         }
-    if (visc ? !PAIRED_VISC : !PAIRED)
-      {
-        if (invert)
-          hipLaunchKernelGGL((k_height_rhs<P, true, R, double, OA>), grid, block, 0, s, args, src_h,
-                             src_q, dst_h);
-        else
-          hipLaunchKernelGGL((k_height_rhs<P, false, R, double, OA>), grid, block, 0, s, args, src_h,
-                             src_q, dst_h);
-      }
     if constexpr (!PAIRED)
       if (!visc)
         {
           if (invert)
-            hipLaunchKernelGGL((k_discharge<P, false, 1, R, OA>), grid, block, 0, s, args, S);
+            hipLaunchKernelGGL((k_stage<P, false, R, 1, OA, 1>), items, block, 0, s, args, H, S);
           else
-            hipLaunchKernelGGL((k_discharge<P, false, 2, R, OA>), grid, block, 0, s, args, S);
+            hipLaunchKernelGGL((k_stage<P, false, R, 1, OA, 2>), items, block, 0, s, args, H, S);
         }
   });
   if (visc)
@@ -266,9 +258,9 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
       else
         {
           if (invert)
-            hipLaunchKernelGGL((k_discharge<P, true, 1, R>), grid, block, 0, s, O, S);
+            hipLaunchKernelGGL((k_stage<P, true, R, 1, OpArgs, 1>), items, block, 0, s, O, H, S);
           else
-            hipLaunchKernelGGL((k_discharge<P, true, 2, R>), grid, block, 0, s, O, S);
+            hipLaunchKernelGGL((k_stage<P, true, R, 1, OpArgs, 2>), items, block, 0, s, O, H, S);
         }
     }
   HIP_TRY(hipGetLastError());

@@ -169,8 +169,7 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
 #pragma unroll
     for (int k = 0; k < N1; ++k)
       acc[cc][k] = 0;
-  // two points per trip fill each other's waits; p = 4 has no registers for it (M^-1 L of 25,538
-  // cells FP64 45.3 -> 46.5 us).  RK4 step of 97,280 cells at p = 3 FP64 321 -> 314 us, channel of
+  // two points per trip fill each other's waits; p = 4 has no registers for it.  RK4 step of 97,280 cells at p = 3 FP64 321 -> 314 us, channel of
   // 2,500 at p = 2 70.5 -> 69 us, viscous of 51,200 at p = 2 119 -> 116 us
   constexpr int POINTS = P <= 3 ? 2 : 1;
   // the bed of the next point is loaded one point ahead
@@ -244,8 +243,7 @@ __device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int b
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P), NG = P + 2;
   constexpr bool COMPACT = std::is_same<R, float>::value;
   constexpr int NS = COMPACT ? 1 : 2;  // subfaces integrated in the face loop
-  // FP64 at p = 4: 256 registers do not hold both subfaces' traces (M^-1 L: 318 with both, 288 one
-  // by one; 46.5 us of 25,538 cells either way)
+  // FP64 at p = 4: 256 registers do not hold both subfaces' traces
   constexpr bool ONE_BY_ONE = NS == 2 && P >= 4;
   const R zcr = R(zc);
   // stage input in its centred FP32 form (FP32 stage only; c32_values, c32_centres)
@@ -863,10 +861,9 @@ __device__ __forceinline__ Phys<R, OA::FLAT> physics(const OA &O)
   return {R(O.g), R(O.cu4), R(O.nu)};
 }
 
-// L_zeta (INVERT: M^-1 L_zeta, for apply())
-// KT: storage type of dst (a stage's k vector is stored in R, a caller vector in FP64)
-template <int P, bool INVERT, typename R, typename KT = double, typename OA = OpArgs>
-__global__ __launch_bounds__(CB) void k_height_rhs(OA O, const double *__restrict__ src_h,
+// L_zeta of a split stage into a k vector (stored in R)
+template <int P, typename R>
+__global__ __launch_bounds__(CB) void k_height_rhs(OpArgs O, const double *__restrict__ src_h,
                                                    const double *__restrict__ src_q,
                                                    double *__restrict__ dst)
 {
@@ -884,11 +881,9 @@ __global__ __launch_bounds__(CB) void k_height_rhs(OA O, const double *__restric
   R Racc[1][ND];
   height_operator<P, R>(O, T, M, batch, lane, hx, hy, (const R *)Z, (const R *)QX,
                         (const R *)QY, zc, src_h, src_q, Racc);
-  if (INVERT)
-    tensor_inverse<P>(T, Racc[0], R(1) / (hx * hy));
 #pragma unroll
   for (int k = 0; k < ND; ++k)
-    reinterpret_cast<KT *>(dst)[vix(batch, 1, 0, ND, k, lane)] = KT(Racc[0][k]);
+    reinterpret_cast<R *>(dst)[vix(batch, 1, 0, ND, k, lane)] = Racc[0][k];
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1379,8 +1374,8 @@ __device__ __forceinline__ void discharge_block(const OA &O, const StageArgs &S,
     }
 }
 
-template <int P, bool VISC, int MODE, typename R, typename OA = OpArgs>
-__global__ __launch_bounds__(CB) void k_discharge(OA O, StageArgs S)
+template <int P, bool VISC, int MODE, typename R>
+__global__ __launch_bounds__(CB) void k_discharge(OpArgs O, StageArgs S)
 {
   __shared__ R lds[discharge_lds_words<P, VISC>()];
   discharge_block<P, VISC, MODE, R>(
@@ -2175,7 +2170,7 @@ __device__ __forceinline__ void height_stage_block(const OA &O, const StageArgs 
     {
       const double hx = O.hxy[((size_t)batch * 2) * CB + lane];
       const double hy = O.hxy[((size_t)batch * 2 + 1) * CB + lane];
-      area = hx * hy;
+      area = MODE == 0 ? hx * hy : double(R(hx) * R(hy));
       R Zo[ND], QX[ND], QY[ND];
       const double zc = load_own<P, R>(S.src_h, S.src_q, batch, lane, Zo, QX, QY);
       height_operator<P, R>(O, basis<R>(P), physics<R>(O), batch, lane, R(hx), R(hy),
@@ -2284,7 +2279,7 @@ __host__ __device__ constexpr int height_lds_words()
 // slice followed by a discharge slice, each of its own size (mixed p = 4, WPB = 2: 29 KiB per
 // workgroup, five per CU, against 38 KiB and four with two discharge-sized slices).  With
 // WPB = 1 each workgroup holds one discharge-sized slice, whatever kind its item is.
-template <int P, bool VISC, typename R, int WPB, typename OA = OpArgs>
+template <int P, bool VISC, typename R, int WPB, typename OA = OpArgs, int MODE = 0>
 __global__ __launch_bounds__(CB * WPB, (stage_min_waves<P, VISC, R>())) void k_stage(
   OA O, StageArgs H, StageArgs Q)
 {
@@ -2301,9 +2296,9 @@ __global__ __launch_bounds__(CB * WPB, (stage_min_waves<P, VISC, R>())) void k_s
   const int kind = item_kind(w);
   R *slice = WPB == 1 ? lds : lds + (wave / 2) * (HW + DW) + (kind ? HW : 0);
   if (kind)
-    discharge_block<P, VISC, 0, R>(O, Q, w >> 1, slice);
+    discharge_block<P, VISC, MODE, R>(O, Q, w >> 1, slice);
   else
-    height_stage_block<P, R>(O, H, w >> 1, reinterpret_cast<float *>(slice));
+    height_stage_block<P, R, false, false, MODE>(O, H, w >> 1, reinterpret_cast<float *>(slice));
 }
 
 // LDS offset (words of R) of the paired items' exchange area inside the height wave's slice:
