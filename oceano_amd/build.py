@@ -4,12 +4,20 @@ The library holds the host set-up (mesh builder, test-case functions, operator s
 the hand-written HIP kernels; everything is compiled by hipcc into one shared object next
 to this file, so it travels with the repository snapshot.
 """
+import glob
 import os
+import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
+if ROOT not in sys.path:  # run as a program
+    sys.path.insert(0, ROOT)
+
+from oceano_amd.check_code import partial_copies  # noqa: E402
+
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liboceano_dg.so")
 
@@ -45,26 +53,41 @@ def _headers():
 
 
 def build(verbose=False, extra=(), incremental=False):
-    """Compile every source (incremental=True skips objects newer than their inputs)."""
+    """Compile every source (incremental=True skips objects newer than their inputs) and search
+    the device assembly of each for copies that miss lanes (check_code.py)."""
     objs = []
-    os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
+    objdir = os.path.join(HERE, "_build")
+    os.makedirs(objdir, exist_ok=True)
     procs = []
     newest_header = _headers()
-    for src, flags, name in SOURCES:
-        path = os.path.join(CSRC, src)
-        obj = os.path.join(HERE, "_build", name + ".o")
-        if (incremental and os.path.exists(obj)
-                and os.path.getmtime(obj) > max(os.path.getmtime(path), newest_header)):
+    with tempfile.TemporaryDirectory(dir=objdir) as work:
+        for src, flags, name in SOURCES:
+            path = os.path.join(CSRC, src)
+            obj = os.path.join(objdir, name + ".o")
             objs.append(obj)
-            continue
-        cmd = [HIPCC, *COMMON, *flags, *extra, "-x", "hip", "-c", path, "-o", obj]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        procs.append((src, subprocess.Popen(cmd)))
-        objs.append(obj)
-    failed = [src for src, p in procs if p.wait() != 0]
-    if failed:
-        raise RuntimeError("hipcc failed for " + ", ".join(failed))
+            if (incremental and os.path.exists(obj)
+                    and os.path.getmtime(obj) > max(os.path.getmtime(path), newest_header)):
+                continue
+            # a directory each: the degrees' temporary files have the same names
+            part = os.path.join(work, name)
+            os.makedirs(part)
+            cmd = [HIPCC, *COMMON, *flags, *extra, "--save-temps=obj", "-x", "hip", "-c", path,
+                   "-o", os.path.join(part, name + ".o")]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            procs.append((src, name, part, obj, subprocess.Popen(cmd)))
+        failed = [src for src, _, _, _, p in procs if p.wait() != 0]
+        if failed:
+            raise RuntimeError("hipcc failed for " + ", ".join(failed))
+        for src, name, part, obj, _ in procs:
+            (asm,) = glob.glob(os.path.join(part, "*-hip-amdgcn-*.s"))
+            with open(asm) as f:
+                partial = partial_copies(f)
+            if partial:
+                raise RuntimeError("%s: register copies ahead of the instruction that switches "
+                                   "lanes on (oceano_amd/check_code.py) in %s" %
+                                   (src, ", ".join("%s %s" % p[:2] for p in partial)))
+            shutil.move(os.path.join(part, name + ".o"), obj)
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "-shared", "--offload-arch=gfx950", "-fPIC", *objs, "-o", tmp]
     if verbose:

@@ -215,11 +215,12 @@ int launch_rhs_apply(oc_dg *op, const OpArgs &O, bool invert, const double *src_
   S.src_q = src_q;
   S.src_v = src_v;
   S.dst = dst_q;
-  // FP64: one launch of paired items where its registers allow (p <= 3, viscous p <= 2).  Past that
-  // its waves need more than the 256 registers that hold both equations' integrals (p = 4: 288 to
-  // 318, viscous 378): then, and for the FP32 integrals, whose results carry the order of summation
-  // of the unpaired items, one launch of unpaired items. M^-1 L of 25,538 cells at p = 4 52 us
-  // (two launches, one an equation, 77; paired 46.5).
+  // FP64: one launch of paired items at p <= 3, viscous at p <= 2 (as the viscous stage).  At p = 4,
+  // M^-1 L of 25,538 cells, they measured 46.5 us, but the compiler left two of their builds with
+  // register copies that miss the coarse cells of hanging faces (oceano_amd/check_code.py; both wave
+  // roles are short of scalar and of vector registers there).  There, and for the FP32 integrals, whose
+  // results carry the order of summation of the unpaired items, one launch of unpaired items: 52 us
+  // (two launches, one an equation, 77).
   constexpr bool PAIRED = std::is_same<R, double>::value && P <= 3;
   constexpr bool PAIRED_VISC = std::is_same<R, double>::value && P <= 2;
   StageArgs H = S;

@@ -1,0 +1,60 @@
+"""The search of the device assembly for register copies that miss lanes (oceano_amd/check_code.py)."""
+import pytest
+
+from oceano_amd.check_code import partial_copies
+
+# the block at fault, as the compiler wrote it, and its surroundings
+SIDE = """_Zkernel:
+; %bb.0:
+\tv_mov_b32_e32 v1, v0
+\ts_and_saveexec_b64 s[0:1], s[20:21]
+\ts_xor_b64 s[0:1], exec, s[0:1]
+\ts_cbranch_execz .LBB0_2
+; %bb.1:
+\tv_add_f64 v[184:185], v[184:185], v[2:3]
+.LBB0_2:
+HEAD; %bb.3:
+\tv_add_f64 v[184:185], v[184:185], v[4:5]
+.LBB0_4:
+\ts_or_b64 exec, exec, s[0:1]
+\ts_endpgm
+.Lfunc_end0:
+"""
+COPIES = "\tv_accvgpr_write_b32 a38, v184\n\tv_accvgpr_write_b32 a39, v185\n"
+SCALAR = "\ts_mov_b64 s[72:73], s[54:55]\n"
+READ_LANE = "\tv_readlane_b32 s56, v251, 17\n"
+ON = "\ts_or_saveexec_b64 s[0:1], s[0:1]\n"
+OFF = "\ts_xor_b64 exec, exec, s[0:1]\n\ts_cbranch_execz .LBB0_4\n"
+ON_OFF = "\ts_andn2_saveexec_b64 s[0:1], s[0:1]\n\ts_cbranch_execz .LBB0_4\n"
+
+
+@pytest.mark.parametrize("head,found", [
+    (COPIES + SCALAR + ON + OFF, True),
+    (COPIES + SCALAR + ON_OFF, True),
+    ("\tv_mov_b64_e32 v[8:9], v[184:185]\n" + SCALAR + ON + OFF, True),
+    ("\tscratch_store_dwordx2 off, v[184:185], off\n" + ON + OFF, True),
+    (SCALAR + ON + COPIES + OFF, False),
+    (SCALAR + READ_LANE + ON_OFF, False),
+    ("\tv_cmp_lt_i32_e32 vcc, 1, v46\n" + ON_OFF, False),
+])
+def test_else_block(head, found):
+    got = partial_copies(SIDE.replace("HEAD", head).splitlines(True))
+    assert [g[:2] for g in got] == ([("_Zkernel", ".LBB0_2")] if found else [])
+
+
+@pytest.mark.parametrize("first,found", [("", True), ("\tv_add_f64 v[8:9], v[2:3], v[4:5]\n", False)])
+def test_block_entered_from_above(first, found):
+    """without the skip a block follows the side that ran: its own work may stand there"""
+    text = SIDE.replace("HEAD", first + COPIES + SCALAR + ON + OFF)
+    text = text.replace("\ts_cbranch_execz .LBB0_2\n", "")
+    got = partial_copies(text.replace(".LBB0_2:", "; %bb.2:").splitlines(True))
+    assert [g[:2] for g in got] == ([("_Zkernel", "%bb.2")] if found else [])
+
+
+def test_end_of_a_branch():
+    text = SIDE.replace("HEAD", ON + OFF).replace(".LBB0_4:\n", ".LBB0_4:\n" + COPIES + SCALAR)
+    assert [g[:2] for g in partial_copies(text.splitlines(True))] == [("_Zkernel", ".LBB0_4")]
+    # skips are a kernel's own
+    other = text.replace("_Zkernel", "_Zother").replace("s_cbranch_execz .LBB0_4", "s_nop 0")
+    got = partial_copies((text + other).splitlines(True))
+    assert [g[:2] for g in got] == [("_Zkernel", ".LBB0_4")]
