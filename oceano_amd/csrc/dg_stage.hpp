@@ -169,9 +169,14 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
 #pragma unroll
     for (int k = 0; k < N1; ++k)
       acc[cc][k] = 0;
-  // two points per trip fill each other's waits; p = 4 has no registers for it.  RK4 step of 97,280 cells at p = 3 FP64 321 -> 314 us, channel of
-  // 2,500 at p = 2 70.5 -> 69 us, viscous of 51,200 at p = 2 119 -> 116 us
-  constexpr int POINTS = P <= 3 ? 2 : 1;
+  // Two points per trip fill each other's waits where the registers hold both.  RK4 step of 97,280
+  // cells at p = 3 FP64 321 -> 314 us, channel of 2,500 at p = 2 70.5 -> 69 us, viscous of 51,200 at
+  // p = 2 119 -> 116 us; FP32 with a stored bed, 24,000 cells: p = 1 50.6 -> 48.5, p = 2 90.4 -> 89,
+  // p = 3 139 -> 140.5 us.  At p = 4 they do not, nor in FP64 at p = 3 beside a stored bed's loads:
+  // the stage kernels spilled up to 300 registers there, with one point at most 3.  24,000 cells,
+  // two points -> one: bed and friction 258 -> 200 us a step (97,000 cells 511 -> 392), unpaired items
+  // 430 -> 182, wind and Coriolis over a flat bed 261 -> 213, viscous 245 -> 193, additive 286 -> 225.
+  constexpr int POINTS = P <= 2 || (P == 3 && (FLAT || !std::is_same<R, double>::value)) ? 2 : 1;
   // the bed of the next point is loaded one point ahead
   const size_t fz0 = (size_t)fi * NG * 2;
   R zb_next[2];

@@ -1,6 +1,14 @@
-"""The search of the device assembly for register copies that miss lanes (oceano_amd/check_code.py)."""
+"""The compiled kernels: the search of their assembly for register copies that miss lanes
+(oceano_amd/check_code.py), and what they spill."""
+import glob
+import os
+import re
+import shutil
+import subprocess
+
 import pytest
 
+from oceano_amd.build import LIB
 from oceano_amd.check_code import partial_copies
 
 # the block at fault, as the compiler wrote it, and its surroundings
@@ -58,3 +66,32 @@ def test_end_of_a_branch():
     other = text.replace("_Zkernel", "_Zother").replace("s_cbranch_execz .LBB0_4", "s_nop 0")
     got = partial_copies((text + other).splitlines(True))
     assert [g[:2] for g in got] == [("_Zkernel", ".LBB0_4")]
+
+
+OBJDUMP, READELF = ("/opt/rocm/llvm/bin/llvm-" + t for t in ("objdump", "readelf"))
+
+
+def _spilled(tmp_path):
+    """{kernel: vector registers it spills}, from the metadata of the built library"""
+    shutil.copy(LIB, tmp_path)
+    subprocess.run([OBJDUMP, "--offloading", os.path.basename(LIB)], cwd=tmp_path, check=True,
+                   stdout=subprocess.DEVNULL)
+    out = {}
+    for part in glob.glob(str(tmp_path / "*gfx950")):
+        notes = subprocess.run([READELF, "--notes", part], check=True, stdout=subprocess.PIPE,
+                               text=True).stdout
+        for kernel in notes.split("  - .agpr_count")[1:]:
+            name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
+            out[name] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1))
+    return out
+
+
+@pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(READELF)),
+                    reason="no ROCm tools")
+def test_fp64_stage_kernels_keep_their_registers(tmp_path):
+    """FP64 stage, M^-1 L, L and additive kernels at p = 3 (every terms type, paired or not): the few
+    registers of a loop's bookkeeping may be spilled, not its work"""
+    spilled = {k: v for k, v in _spilled(tmp_path).items()
+               if re.search(r"k_stage(_pair|_ark_pair)?ILi3E(Lb[01]E)?d", k)}
+    assert len(spilled) >= 20
+    assert max(spilled.values()) <= 4, {k: v for k, v in spilled.items() if v > 4}
