@@ -177,15 +177,22 @@ __device__ __forceinline__ void subface_integral(const Basis<R> &T, const FieldV
   // two points -> one: bed and friction 258 -> 200 us a step (97,000 cells 511 -> 392), unpaired items
   // 430 -> 182, wind and Coriolis over a flat bed 261 -> 213, viscous 245 -> 193, additive 286 -> 225.
   constexpr int POINTS = P <= 2 || (P == 3 && (FLAT || !std::is_same<R, double>::value)) ? 2 : 1;
-  // the bed of the next point is loaded one point ahead
+  // The bed of the next point is loaded one point ahead, but not in FP32 at p = 4, where the two
+  // waves of a SIMD cover the load (FP64 has one).  24,000 cells at p = 4, ahead -> at the point: FP32
+  // general 356 -> 351 us a step, viscous 256 -> 251; FP64 bed and friction 297 -> 308, general 397 ->
+  // 412.
+  constexpr bool AHEAD = P <= 3 || std::is_same<R, double>::value;
   const size_t fz0 = (size_t)fi * NG * 2;
   R zb_next[2];
-  fld_row<2, 1>(fz, fz0, zb_next);
+  if (AHEAD)
+    fld_row<2, 1>(fz, fz0, zb_next);
 #pragma unroll POINTS
   for (int a = 0; a < NG; ++a)
     {
+      if (!AHEAD)
+        fld_row<2, 1>(fz, fz0 + 2 * a, zb_next);
       const R zbm = zb_next[0], zbp = zb_next[1];
-      if (a + 1 < NG)
+      if (AHEAD && a + 1 < NG)
         fld_row<2, 1>(fz, fz0 + 2 * (a + 1), zb_next);
       R zo = 0, xo = 0, yo = 0, zn = 0, xn = 0, yn = 0;
 #pragma unroll
