@@ -265,10 +265,10 @@ struct FieldV<R, true>
   R cval;
 };
 
-template <typename R, typename OA>
-__device__ __forceinline__ FieldV<R, OA::FLAT> in_vgprs(const OA &, const Field &f)
+template <typename R, bool FLAT>
+__device__ __forceinline__ FieldV<R, FLAT> in_vgprs(const Field &f)
 {
-  if constexpr (OA::FLAT)
+  if constexpr (FLAT)
     return {R(f.cval)};
   else
     {
@@ -276,6 +276,11 @@ __device__ __forceinline__ FieldV<R, OA::FLAT> in_vgprs(const OA &, const Field 
       asm volatile("" : "+v"(v.ptr), "+v"(v.cval));
       return v;
     }
+}
+template <typename R, typename OA>
+__device__ __forceinline__ FieldV<R, OA::FLAT> in_vgprs(const OA &, const Field &f)
+{
+  return in_vgprs<R, OA::FLAT>(f);
 }
 
 template <typename R>

@@ -985,12 +985,12 @@ __device__ __forceinline__ void pair_exchange(R (&A)[3][(P + 1) * (P + 1)], R *x
 // cell term of L_q (advective and diffusive flux, gravity, Manning friction, wind stress,
 // Coriolis; OceanDG.h:696-743, ShallowWater.h:381-432): AX, AY += the integrals against
 // grad(phi) and phi.  The batch's own zeta (deviation from zcr), q (and velocity) are read
-// from the lane-interleaved LDS copy `lds`.
-template <int P, bool VISC, typename R, typename OA>
-__device__ __forceinline__ void discharge_cell_term(const OA &O, const Basis<R> &T,
-                                                    const R *lds, int batch, int lane, R hx,
-                                                    R hy, R zcr, R (&AX)[(P + 1) * (P + 1)],
-                                                    R (&AY)[(P + 1) * (P + 1)])
+// from the lane-interleaved LDS copy `lds`.  FLAT: the bed is uniform.
+template <int P, bool VISC, bool FLAT, typename R, typename OA>
+__device__ __forceinline__ void discharge_rows(const OA &O, const Basis<R> &T, const R *lds,
+                                               int batch, int lane, R hx, R hy, R zcr,
+                                               R (&AX)[(P + 1) * (P + 1)],
+                                               R (&AY)[(P + 1) * (P + 1)])
 {
   constexpr int N1 = P + 1, ND = N1 * N1, NQ = nq_of(P);
   const LdsVec<R> Z{lds + lane}, QX{lds + ND * CB + lane}, QY{lds + 2 * ND * CB + lane};
@@ -999,7 +999,7 @@ __device__ __forceinline__ void discharge_cell_term(const OA &O, const Basis<R> 
   const R g = R(O.g), nu = R(O.nu);
   const R ihx = R(1) / hx, ihy = R(1) / hy, area = hx * hy;
   const size_t c0base = (size_t)batch * NQ * NQ * CB + lane;
-  const auto bed = in_vgprs<R>(O, O.cell0[0]);
+  const auto bed = in_vgprs<R, FLAT>(O.cell0[0]);
 #pragma unroll 1
   for (int b = 0; b < NQ; ++b)
     {
@@ -1132,6 +1132,26 @@ __device__ __forceinline__ void discharge_cell_term(const OA &O, const Basis<R> 
             AY[i + N1 * j] += two_products(T.Sq[b][j], WSY[i], T.Dq[b][j], WDY[i]);
           }
     }
+}
+
+// Where no term is known when the kernel is compiled, the bed can still be uniform (wind and
+// Coriolis force over a flat bed, viscosity alone).  Asked at every row, that ends a basic block; in FP32 the
+// rows exist twice instead and are chosen once.  24,000 cells, mixed: wind and Coriolis over a flat
+// bed, p = 2 90 -> 85 us a step, p = 3 149 -> 147; viscous p = 2 98 -> 94, p = 3 146 -> 144; with a stored
+// bed, p = 2 117 -> 111.  FP64 has no registers for it (wind and Coriolis at p = 4 352 -> 365).
+template <int P, bool VISC, typename R, typename OA>
+__device__ __forceinline__ void discharge_cell_term(const OA &O, const Basis<R> &T,
+                                                    const R *lds, int batch, int lane, R hx,
+                                                    R hy, R zcr, R (&AX)[(P + 1) * (P + 1)],
+                                                    R (&AY)[(P + 1) * (P + 1)])
+{
+  if constexpr (std::is_same<OA, OpArgs>::value && centred<R>())
+    if (!O.cell0[0].ptr)
+      {
+        discharge_rows<P, VISC, true>(O, T, lds, batch, lane, hx, hy, zcr, AX, AY);
+        return;
+      }
+  discharge_rows<P, VISC, OA::FLAT>(O, T, lds, batch, lane, hx, hy, zcr, AX, AY);
 }
 
 // IN32 (FP32 paired stage): the stage input S.src_h, S.src_q comes in its centred FP32 form
