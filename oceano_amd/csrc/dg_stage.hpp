@@ -1475,22 +1475,13 @@ __device__ __forceinline__ int depth_mass(const OpArgs &O, const DegreeTables &T
   return ndry;
 }
 
-// Z += Dinv R; returns the update's l1 norm.  R is advanced to the new Z by the linear
-// formula R <- R - area (M1 x M1) dZ (the next residual while the depth is linear in Z)
-template <int P, typename DinvFn>
-__device__ __forceinline__ double jacobi_update(const DegreeTables &T, double area, double *R,
-                                                double *Z, DinvFn dinv)
+// R <- R - area (M1 x M1) dZ: the residual advanced to Z + dZ while the depth is linear in Z
+template <int P>
+__device__ __forceinline__ void advance_residual(const DegreeTables &T, double area,
+                                                 double (&R)[(P + 1) * (P + 1)],
+                                                 double (&dZ)[(P + 1) * (P + 1)])
 {
-  constexpr int N1 = P + 1, ND = N1 * N1;
-  double dZ[ND], norm = 0.0;
-#pragma unroll
-  for (int i = 0; i < ND; ++i)
-    {
-      const double old = Z[i];
-      Z[i] += dinv(i) * R[i];
-      dZ[i] = Z[i] - old;
-      norm += fabs(dZ[i]);
-    }
+  constexpr int N1 = P + 1;
 #pragma unroll
   for (int l = 0; l < N1; ++l)
     {
@@ -1519,18 +1510,6 @@ __device__ __forceinline__ double jacobi_update(const DegreeTables &T, double ar
           s += T.M1[j][l] * dZ[i + N1 * l];
         R[i + N1 * j] -= area * s;
       }
-  return norm;
-}
-
-// one sweep of a cell that is wet at every GL point, with the full lumped mass
-template <int P>
-__device__ __forceinline__ double linear_sweep(const DegreeTables &T, double area,
-                                               double inv_area, double *R, double *Z)
-{
-  constexpr int N1 = P + 1;
-  return jacobi_update<P>(T, area, R, Z, [&](int i) {
-    return T.ilumped2[i % N1][i / N1] * inv_area;
-  });
 }
 
 // Jacobi solve of one cell: Z holds zeta^n on entry (and the dry lift is applied to it),
@@ -1594,7 +1573,25 @@ __device__ __forceinline__ int jacobi_solve(const OpArgs &O, const DegreeTables 
   double norm = 1.0, hbase = -1.0, C = 0.0;
   bool linear = false;
   double Rr[ND];
-  auto update = [&](auto dinv) { C += norm = jacobi_update<P>(T, area, Rr, Z, dinv); };
+  // Z += Dinv Rr and its l1 norm; the residual is advanced to the new Z by the linear
+  // formula (used only if the next sweep is certified linear, recomputed otherwise).  Written out
+  // here: as a function that returned the norm it took the FP32 kernels that inline this solve 14
+  // to 32 registers more (viscous stage at p = 3: one wave per SIMD instead of two, 525 -> 674 us for
+  // five steps of 51,200 cells)
+  auto update = [&](auto dinv) {
+    norm = 0.0;
+    double dZ[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      {
+        const double old = Z[i];
+        Z[i] += dinv(i) * Rr[i];
+        dZ[i] = Z[i] - old;
+        norm += fabs(dZ[i]);
+      }
+    C += norm;
+    advance_residual<P>(T, area, Rr, dZ);
+  };
   auto wet_dinv = [&](int i) { return T.ilumped2[i % N1][i / N1] * inv_area; };
   int k = 0;
   for (; k < O.max_it && norm > 1e-12; ++k)
@@ -1714,8 +1711,8 @@ __device__ __forceinline__ double least_depth(const OA &O, const DegreeTables &T
 template <int P>
 __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &T,
                                            const Phys<double> &M, int batch, int lane,
-                                           double area, double *r, double *Z, double hmin,
-                                           double *front)
+                                           double area, double (&r)[(P + 1) * (P + 1)],
+                                           double *Z, double hmin, double *front)
 {
   constexpr int N1 = P + 1, ND = N1 * N1;
   if (front)
@@ -1793,7 +1790,19 @@ __device__ __forceinline__ int depth_solve(const OpArgs &O, const DegreeTables &
       double norm = 1.0;
 #pragma unroll 1
       for (; k < O.max_it && norm > 1e-12; ++k)
-        norm = linear_sweep<P>(T, area, inv_area, r, Z);
+        {
+          norm = 0.0;
+          double dZ[ND];
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            {
+              const double old = Z[i];
+              Z[i] += T.ilumped2[i % N1][i / N1] * inv_area * r[i];
+              dZ[i] = Z[i] - old;
+              norm += fabs(dZ[i]);
+            }
+          advance_residual<P>(T, area, r, dZ);
+        }
       return k;
     }
   unsigned long long bits = 0;

@@ -71,8 +71,8 @@ def test_end_of_a_branch():
 OBJDUMP, READELF = ("/opt/rocm/llvm/bin/llvm-" + t for t in ("objdump", "readelf"))
 
 
-def _spilled(tmp_path):
-    """{kernel: vector registers it spills}, from the metadata of the built library"""
+def _registers(tmp_path):
+    """{kernel: (vector registers it uses, those it spills)}, from the built library's metadata"""
     shutil.copy(LIB, tmp_path)
     subprocess.run([OBJDUMP, "--offloading", os.path.basename(LIB)], cwd=tmp_path, check=True,
                    stdout=subprocess.DEVNULL)
@@ -82,16 +82,35 @@ def _spilled(tmp_path):
                                text=True).stdout
         for kernel in notes.split("  - .agpr_count")[1:]:
             name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
-            out[name] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1))
+            out[name] = tuple(int(re.search(r"\.vgpr_%scount:\s+(\d+)" % what, kernel).group(1))
+                              for what in ("", "spill_"))
     return out
 
 
-@pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(READELF)),
-                    reason="no ROCm tools")
+tools = pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(READELF)),
+                           reason="no ROCm tools")
+
+
+@tools
 def test_fp64_stage_kernels_keep_their_registers(tmp_path):
     """FP64 stage, M^-1 L, L and additive kernels at p = 3 (every terms type, paired or not): the few
     registers of a loop's bookkeeping may be spilled, not its work"""
-    spilled = {k: v for k, v in _spilled(tmp_path).items()
+    spilled = {k: v[1] for k, v in _registers(tmp_path).items()
                if re.search(r"k_stage(_pair|_ark_pair)?ILi3E(Lb[01]E)?d", k)}
     assert len(spilled) >= 20
     assert max(spilled.values()) <= 4, {k: v for k, v in spilled.items() if v > 4}
+
+
+@tools
+@pytest.mark.parametrize("kernel,most,spills", [
+    (r"k_stageILi3ELb1Ef\w*OpArgsELi0E", 256, 0),     # viscous stage: two waves per SIMD
+    (r"k_stageILi2ELb1Ef\w*OpArgsELi0E", 128, 0),     # four
+    (r"k_stage_pairILi2EfLb[01]ELb0ELi0E", 128, 0),
+    (r"k_height_jacobiILi[12]E", 128, 0),
+    (r"k_height_jacobiILi3E", 256, 0),
+    (r"k_depth_deferredILi3E", 256, 0)])
+def test_kernels_with_the_sweeps_keep_their_waves(tmp_path, kernel, most, spills):
+    """FP32 kernels that hold the FP64 sweeps of dry cells, and the split path's depth solve"""
+    got = {k: v for k, v in _registers(tmp_path).items() if re.search(kernel, k)}
+    assert got
+    assert all(v[0] <= most and v[1] <= spills for v in got.values()), got
