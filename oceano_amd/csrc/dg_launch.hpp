@@ -115,11 +115,19 @@ int launch_stage(oc_dg *op, const OpArgs &O, uint32_t stage, const double *facto
           // paired in FP64 at p <= 2 (RK4 step of 12,800 cells at p = 1 43 -> 35 us, of 51,200 at
           // p = 2 138 -> 129 us); at p >= 3 the cell term's gradients of the velocity fill two
           // waves' registers and the unpaired items at one wave per SIMD are faster (26,000 hanging
-          // cells at p = 3: 196 us a step, paired 225; 5,000 at p = 4: 264, paired 279)
+          // cells at p = 3: 196 us a step, paired 225; 5,000 at p = 4: 264, paired 279).  FP32 items
+          // are unpaired, by the terms there are: 110,000 cells over a flat bed p = 1 103 -> 94 us a
+          // step, p = 2 185 -> 168, p = 3 343 -> 310, p = 4 749 -> 654 (FP64 at p >= 3 tests them
+          // at run time: there the viscous terms fill the registers either way)
           if constexpr (std::is_same<R, double>::value && P <= 2)
             with_terms(O, [&](auto args) {
               hipLaunchKernelGGL((k_stage_pair<P, R, false, true, 0, decltype(args)>), grid,
                                  dim3(2 * CB), 0, s, args, H, Q);
+            });
+          else if constexpr (std::is_same<R, float>::value)
+            with_terms(O, [&](auto args) {
+              hipLaunchKernelGGL((k_stage<P, true, R, 1, decltype(args)>), dim3(items), block, 0, s,
+                                 args, H, Q);
             });
           else
             hipLaunchKernelGGL((k_stage<P, true, R, 1>), dim3(items), block, 0, s, O, H, Q);
