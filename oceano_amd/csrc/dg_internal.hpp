@@ -66,8 +66,8 @@ struct oc_dg
   float *d_kinv = nullptr;  // mixed precision: momentum inverse mass (unit cell)
   unsigned long long *d_defer = nullptr;  // mixed precision: per batch, deferred lanes
   double *d_post = nullptr; // per-batch results of the reductions [NB]
-  // arguments of a multi-operator stage launch this operator leads (written by a kernel)
-  oceano::MultiArgs *d_multi_args = nullptr;
+  // MultiArgs of a multi-operator stage launch this operator leads (written by a kernel)
+  unsigned char *d_multi_args = nullptr;
   double wet_margin = 10.0;
   // learned closure (oc_dg_set_closure): network (not owned), per-cell sub-grid statistics
   // [batch][3][lane], modal<->nodal tables [nd][nd], correction buffer [batch][2][nd][lane]

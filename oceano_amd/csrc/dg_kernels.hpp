@@ -168,14 +168,16 @@ struct StageArgs
 
 // the arguments of one multi-operator stage launch (dg_stage_multi.hip)
 constexpr int MAXG = OC_MULTI_MAX_OPERATORS;
+template <typename OA>
 struct MultiArgs
 {
   int n_groups;
   int start[MAXG + 1];  // first workgroup of each group; start[n_groups] = grid size
   int degree[MAXG];
-  OpArgs O[MAXG];
+  OA O[MAXG];
   StageArgs H[MAXG], Q[MAXG];
 };
+static_assert(sizeof(PlainArgs) == sizeof(OpArgs), "one buffer holds either block");
 
 __host__ __device__ constexpr int nq_of(int p) { return (3 * p) / 2 + 1; }
 

@@ -967,7 +967,7 @@ int oc_dg_create(const oc_mesh_desc *mesh, const oc_params *prm, oc_dg **out)
       (rc = upload(&op->d_jmat, jacobi_matrix(op->P, op->max_it))) ||
       (rc = upload(&op->d_kinv, inverse_mass_matrix(op->P))) ||
       (rc = dalloc(&op->d_defer, (size_t)NB)) || (rc = dalloc(&op->d_post, (size_t)NB)) ||
-      (rc = dalloc(&op->d_count, 1)) || (rc = dalloc(&op->d_multi_args, 1)))
+      (rc = dalloc(&op->d_count, 1)) || (rc = dalloc(&op->d_multi_args, sizeof(MultiArgs<OpArgs>))))
     {
       free_all(op);
       delete op;

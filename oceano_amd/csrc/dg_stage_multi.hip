@@ -28,17 +28,16 @@ namespace {
 // the stage kernel (in stream order, so a captured graph replays both): the stage kernel
 // reads the group it runs through a pointer, with uniform (scalar) loads.  Indexing the
 // by-value argument block by a run-time group index instead makes the compiler copy the
-// whole block to per-lane scratch memory.  The words are copied by the workgroup's threads from
-// the kernel's argument segment, where A comes first: 4.6 us, against 7.2 us for one thread
-// copying A, ahead of a stage of 51 us.
-__global__ __launch_bounds__(256) void k_put_multi_args(MultiArgs A, MultiArgs *dst)
+// whole block to per-lane scratch memory.  The words are copied by the workgroup's threads:
+// 4.6 us, against 7.2 us for one thread copying A, ahead of a stage of 51 us.
+template <typename OA>
+__global__ __launch_bounds__(256) void k_put_multi_args(MultiArgs<OA> A, MultiArgs<OA> *dst)
 {
-  static_assert(sizeof(MultiArgs) % sizeof(int) == 0, "copied as words");
-  typedef __attribute__((address_space(4))) const int cint;
-  const cint *src = (const cint *)__builtin_amdgcn_kernarg_segment_ptr();
+  static_assert(sizeof(A) % sizeof(int) == 0, "copied as words");
+  const int *src = reinterpret_cast<const int *>(&A);
   int *to = reinterpret_cast<int *>(dst);
 #pragma unroll
-  for (int i = threadIdx.x; i < (int)(sizeof(MultiArgs) / sizeof(int)); i += 256)
+  for (int i = threadIdx.x; i < (int)(sizeof(A) / sizeof(int)); i += 256)
     to[i] = src[i];
 }
 
@@ -60,14 +59,14 @@ constexpr int multi_min_waves()
 
 template <typename R, typename OA>
 __global__ __launch_bounds__(CB, (multi_min_waves<R>())) void k_stage_multi(
-  const MultiArgs *__restrict__ A)
+  const MultiArgs<OA> *__restrict__ A)
 {
   __shared__ R lds[discharge_lds_words<4, false>()];
   const int b = blockIdx.x;
   int g = 0;
   while (g + 1 < A->n_groups && b >= A->start[g + 1])
     ++g;
-  const OA &O = static_cast<const OA &>(A->O[g]);  // the same members
+  const OA &O = A->O[g];
   const int n_items = 2 * O.n_batches;
   const int local = b - A->start[g];
   if (local >= n_items)  // padding of the group's range to a multiple of the XCD count
@@ -111,14 +110,14 @@ __device__ __forceinline__ void multi_pair(const OA &O, const StageArgs &H,
 
 template <typename R, typename OA>
 __global__ __launch_bounds__(2 * CB, (multi_min_waves<R>())) void k_stage_multi_pair(
-  const MultiArgs *__restrict__ A)
+  const MultiArgs<OA> *__restrict__ A)
 {
   __shared__ __align__(16) R lds[pair_lds_words<4, R>()];
   const int b = blockIdx.x;
   int g = 0;
   while (g + 1 < A->n_groups && b >= A->start[g + 1])
     ++g;
-  const OA &O = static_cast<const OA &>(A->O[g]);  // the same members
+  const OA &O = A->O[g];
   const int local = b - A->start[g];
   if (local >= O.n_batches)  // padding of the group's range to a multiple of the XCD count
     return;
@@ -159,35 +158,36 @@ int stage_multi(int n, oc_dg *const *ops, const OpArgs *O, uint32_t stage,
                 double *const *w_h, double *const *w_q, double *const *r_h,
                 double *const *r_q, hipStream_t s)
 {
-  MultiArgs A{};
-  A.n_groups = n;
   // paired items when every operator asks for them (one workgroup per batch), else one
-  // workgroup per work item
-  bool paired = true;
-  for (int g = 0; g < n; ++g)
-    paired = paired && ops[g]->paired_items;
-  int start = 0;
+  // workgroup per work item; the groups share a kernel: flat and free of sources only if all of
+  // them are
+  bool paired = true, plain = true;
   for (int g = 0; g < n; ++g)
     {
-      A.start[g] = start;
-      A.degree[g] = ops[g]->P;
-      A.O[g] = O[g];
-      stage_args(O[g], stage, factor[g], ri_h[g], ri_q[g], nullptr, ki_h[g], ki_q[g], n_ki,
-                 w_h[g], w_q[g], r_h[g], r_q[g], 0, A.H[g], A.Q[g]);
-      const int blocks = paired ? ops[g]->NB : 2 * ops[g]->NB;
-      start += (blocks + NXCD - 1) / NXCD * NXCD;
+      paired = paired && ops[g]->paired_items;
+      plain = plain && is_plain(O[g]);
     }
-  A.start[n] = start;
   const bool mixed = ops[0]->precision == OC_PRECISION_MIXED;
-  MultiArgs *dA = ops[0]->d_multi_args;
-  hipLaunchKernelGGL(k_put_multi_args, dim3(1), dim3(256), 0, s, A, dA);
-  HIP_TRY(hipGetLastError());
-  // the groups share a kernel: flat and free of sources only if all of them are
-  bool plain = true;
-  for (int g = 0; g < n; ++g)
-    plain = plain && is_plain(O[g]);
+  StageArgs H[MAXG];
   auto launch = [&](auto args) {
     using OA = decltype(args);
+    MultiArgs<OA> A{};
+    A.n_groups = n;
+    int start = 0;
+    for (int g = 0; g < n; ++g)
+      {
+        A.start[g] = start;
+        A.degree[g] = ops[g]->P;
+        A.O[g] = OA{O[g]};
+        stage_args(O[g], stage, factor[g], ri_h[g], ri_q[g], nullptr, ki_h[g], ki_q[g], n_ki,
+                   w_h[g], w_q[g], r_h[g], r_q[g], 0, A.H[g], A.Q[g]);
+        H[g] = A.H[g];
+        const int blocks = paired ? ops[g]->NB : 2 * ops[g]->NB;
+        start += (blocks + NXCD - 1) / NXCD * NXCD;
+      }
+    A.start[n] = start;
+    MultiArgs<OA> *dA = reinterpret_cast<MultiArgs<OA> *>(ops[0]->d_multi_args);
+    hipLaunchKernelGGL(k_put_multi_args<OA>, dim3(1), dim3(256), 0, s, A, dA);
     if (paired && mixed)
       hipLaunchKernelGGL((k_stage_multi_pair<float, OA>), dim3(start), dim3(2 * CB), 0, s, dA);
     else if (paired)
@@ -206,7 +206,7 @@ int stage_multi(int n, oc_dg *const *ops, const OpArgs *O, uint32_t stage,
     for (int g = 0; g < n; ++g)
       if (defer_depth_solve(ops[g]->P))
         {
-          StageArgs D = A.H[g];
+          StageArgs D = H[g];
           for (uint32_t j = 0; j <= stage; ++j)
             D.kprev[j] = ki_h[g][j + 1];
           const dim3 dgrid((ops[g]->NB + DEFER_BATCHES - 1) / DEFER_BATCHES);
