@@ -87,7 +87,7 @@ struct OpArgs
   // mixed precision: closed form of max_it linear Jacobi sweeps on a wet unit cell,
   // [nd][nd] row-major (delta = J r / area), and the wet-cell safety factor
   const float *jmat;
-  // the capped sweeps of a wet cell in the eigenbasis of D^-1 M (wet_depth_solve): per
+  // the capped sweeps of a wet cell in the eigenbasis of D^-1 M (depth_solve): per
   // eigen-coefficient the gain of all max_it sweeps [nd] and the decay of the last update
   // whose norm the stop test reads [nd]; the bounds that certify it
   const double *eig;

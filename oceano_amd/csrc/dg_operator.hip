@@ -154,7 +154,7 @@ DegreeTables make_tables(int p)
   return t;
 }
 
-// The capped sweeps of a wet cell in the eigenbasis (wet_depth_solve): with r the right-hand
+// The capped sweeps of a wet cell in the eigenbasis (depth_solve): with r the right-hand
 // side, c = (Ved x Ved) r / area, and mu = 1 - el_a el_b in [0, 1), update k (k = 1, 2, ..) is
 // (Ve x Ve) mu^(k-1) c, so K sweeps add up to (Ve x Ve) gain c with gain = sum_{k<K} mu^k.
 //   tab        gain [nd], then mu^(K-2) [nd] (1 for K < 3)

@@ -565,8 +565,9 @@ __device__ __forceinline__ void face_terms(const OA &O, const Basis<R> &T, int b
 
 // in place: U <- M^-1 U for one component on an affine cell of area 1/inv_area.  FP64: M^-1 =
 // (Kn x Kn) / area in two contractions, 2 (p+1)^3 multiply-adds a component against 4 (p+1)^3
-// and (p+1)^2 divisions through the collocation points; FP32 (p <= 2) keeps the latter, whose
-// rounding the mixed path's results have.  Measured, FP64 RK4 step of 97,280 cells at p = 3:
+// and (p+1)^2 divisions through the collocation points; FP32 (momentum at p <= 2, the height
+// equation's M^-1 L_zeta at every degree) keeps the latter, whose rounding the mixed path's
+// results have.  Measured, FP64 RK4 step of 97,280 cells at p = 3:
 // 379 -> 375 us; apply of 25,538 cells at p = 4: 98.8 -> 94.3 us.
 template <int P>
 __device__ __forceinline__ void tensor_inverse(const Basis<double> &T, double *U,
@@ -1865,8 +1866,8 @@ __device__ __forceinline__ float least_depth32(const OA &O, int batch, int lane,
 // FP32 stage kernel).  Called by the active lanes; lane 0 of a batch is always active.
 // The FP32 stage leaves the FP64 depth solve of cells near the floor to k_depth_deferred
 // at p = 4, where its registers would spill heavily (256 VGPRs, 268 B per lane); at p <= 3
-// the stage kernel does it itself.  At p = 3 that costs 47 spill slots but keeps 3 waves
-// per SIMD, and saves the second launch: measured 2 % faster per stage on the 97k-cell
+// the stage kernel does it itself.  At p = 3 that costs 74 to 103 spilled registers (paired; 58
+// to 70 unpaired), most of them in the sweeps themselves, but keeps 3 waves per SIMD, and saves the second launch: measured 2 % faster per stage on the 97k-cell
 // hanging vortex.
 __host__ __device__ constexpr bool defer_depth_solve(int p) { return p >= 4; }
 
@@ -2105,7 +2106,7 @@ __global__ __launch_bounds__(CB) void k_depth_deferred(OpArgs O, StageArgs S)
 // L_zeta, front and depth solve of one batch of cells in one pass: L_zeta stays in
 // registers for the front (it is also written out as ki_h[stage+1] for later stages).
 // IN32 / S.out32 as for discharge_block (the zeta register's centres included)
-// MODE 1, 2 (paired only): apply and rhs, M^-1 L_zeta or L_zeta into the FP64 vector S.dst
+// MODE 1, 2: apply and rhs, M^-1 L_zeta or L_zeta into the FP64 vector S.dst
 template <int P, typename R, bool PAIR = false, bool IN32 = false, int MODE = 0,
           typename OA = OpArgs>
 __device__ __forceinline__ void height_stage_block(const OA &O, const StageArgs &S,

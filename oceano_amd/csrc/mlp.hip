@@ -72,7 +72,8 @@ __device__ __forceinline__ bf16x8 load_inputs(const float *__restrict__ X, int64
 //
 // The chain of one chunk (eight dependent products, three GELUs) bounds it, not its 150 MFMAs:
 // at 4096 rows every wave has one chunk.  So nothing waits in it that need not: the weights of both
-// directions and the weight gradients stay in registers (one wave per SIMD has 512), and an
+// directions and the weight gradients stay in registers (one wave per SIMD has 512, all used; 60
+// more are spilled), and an
 // accumulator's layout (sample 4 (l / 16) + j, unit 16 ct + l % 16) is already the operand
 // layout of the 16-sample weight-gradient products, so only the row operands of the layer
 // products cross LDS.  4096 rows: about 56 us with weights and gradients in LDS, 26.5 us.
